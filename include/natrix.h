@@ -382,6 +382,10 @@ int nx_conv3x3_wgrad(const void* x, const void* dy, float* dw, float* work, int 
                      int n, int h, int wd, int cin, int cout, void* stream);
 /* dz = dy where y > 0 else 0 (bfloat16, `count` elements) */
 int nx_relu_bwd(const void* y, const void* dy, void* dz, long long count, void* stream);
+/* the same over a (rows x c) matrix, and db[c] (float32) = the column sums of
+ * dz (the bias gradient) from the same pass; work: 1024*c float32 */
+int nx_relu_bwd_colsum(const void* y, const void* dy, void* dz, float* db, float* work,
+                       long long rows, int c, void* stream);
 /* out[c] = sum over rows of a bfloat16 (rows x c) matrix; work: 1024*c float32 */
 int nx_colsum(const void* a, float* out, float* work, long long rows, int c,
               void* stream);

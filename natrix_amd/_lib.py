@@ -173,6 +173,7 @@ SIGNATURES = {
     "nx_conv3x3_dgrad": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "nx_conv3x3_wgrad": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "nx_relu_bwd": [_P, _P, _P, C.c_longlong, _P],
+    "nx_relu_bwd_colsum": [_P, _P, _P, _P, _P, C.c_longlong, _I, _P],
     "nx_colsum": [_P, _P, _P, C.c_longlong, _I, _P],
     "nx_avgpool2": [_P, _P, _I, _I, _I, _I, _I, _P],
     "nx_upsample2": [_P, _P, _I, _I, _I, _I, _I, _P],

@@ -370,103 +370,12 @@ __global__ void k_flip_weights(const uint16_t* __restrict__ w, uint16_t* __restr
   wt[((long long)ci * 9 + (8 - tap)) * Cout + co] = w[i];
 }
 
-// ---------------------------------------------------------------- wgrad
-// dw[co][tap][ci] = sum_m dy[m][co] * x[m shifted by tap][ci]
-// grid: (Cout/64 * Cin/64, 9, splits); block 256 (2x2 waves of 32x32)
-constexpr int WG_CHUNK = 64;
-
-__global__ void __launch_bounds__(256)
-    k_conv3x3_wgrad(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
-                    float* __restrict__ part, int N, int H, int W, int Cin,
-                    int Cout, long long pix_per_split) {
-  __shared__ uint16_t sA[64][WG_CHUNK + 8];  // [co][pixel]
-  __shared__ uint16_t sB[64][WG_CHUNK + 8];  // [ci][pixel]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 31, kb = lane >> 5;
-  const int tiles_ci = (Cin + 63) / 64;
-  const int co0 = (blockIdx.x / tiles_ci) * 64;
-  const int ci0 = (blockIdx.x % tiles_ci) * 64;
-  const int tap = blockIdx.y;
-  const int dy_ = tap / 3 - 1, dx_ = tap % 3 - 1;
-  const long long M = (long long)N * H * W;
-  const long long p_begin = (long long)blockIdx.z * pix_per_split;
-  const long long p_end = p_begin + pix_per_split < M ? p_begin + pix_per_split : M;
-  const int wm = wave >> 1, wn = wave & 1;  // wave's 32x32 quadrant
-  f32x16 acc;
-  for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-  const int hw = H * W;
-  for (long long p0 = p_begin; p0 < p_end; p0 += WG_CHUNK) {
-    // stage: 64 pixels x 64 channels of dy and of the shifted x, 8
-    // channels (one 16-byte load) per thread and pass, zero beyond C
-    for (int it = 0; it < 2; ++it) {
-      const int idx = threadIdx.x + it * 256;
-      const int pl = idx >> 3;         // pixel within chunk (0..63)
-      const int cq = (idx & 7) * 8;    // channel offset (0..56)
-      const long long m = p0 + pl;
-      uint4 va = make_uint4(0, 0, 0, 0), vb = va;
-      if (m < p_end) {
-        if (co0 + cq < Cout)
-          va = *reinterpret_cast<const uint4*>(dy + m * Cout + co0 + cq);
-        const long long img = m / hw;
-        const int rem = (int)(m - img * hw);
-        const int yy = rem / W + dy_, xx = rem % W + dx_;
-        if (ci0 + cq < Cin && yy >= 0 && yy < H && xx >= 0 && xx < W)
-          vb = *reinterpret_cast<const uint4*>(
-              x + (img * hw + (long long)yy * W + xx) * Cin + ci0 + cq);
-      }
-      const uint16_t* ta = reinterpret_cast<const uint16_t*>(&va);
-      const uint16_t* tb = reinterpret_cast<const uint16_t*>(&vb);
-      for (int t = 0; t < 8; ++t) {
-        sA[cq + t][pl] = ta[t];
-        sB[cq + t][pl] = tb[t];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k0 = 0; k0 < WG_CHUNK; k0 += 16) {
-      const bf16x8 a = ld_frag(&sA[wm * 32 + r][k0 + kb * 8]);
-      const bf16x8 b = ld_frag(&sB[wn * 32 + r][k0 + kb * 8]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // partial[split][co][tap][ci]
-  const long long base = (long long)blockIdx.z * Cout * 9 * Cin;
-  for (int e = 0; e < 16; ++e) {
-    const int co = co0 + wm * 32 + 8 * (e >> 2) + 4 * kb + (e & 3);
-    const int ci = ci0 + wn * 32 + r;
-    if (co < Cout && ci < Cin) part[base + ((long long)co * 9 + tap) * Cin + ci] = acc[e];
-  }
-}
-
-// out[i] = sum_s part[s*n + i], fixed order
-__global__ void k_sum_splits(const float* __restrict__ part, float* __restrict__ out,
-                             long long n, int splits) {
-  const long long i = blockIdx.x * 256ll + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.0f;
-  for (int k = 0; k < splits; ++k) s += part[(long long)k * n + i];
-  out[i] = s;
-}
-
 // ---------------------------------------------------------------- elementwise
 __global__ void k_relu_bwd(const uint16_t* __restrict__ y, const uint16_t* __restrict__ dy,
                            uint16_t* __restrict__ dz, long long n) {
   const long long i = blockIdx.x * 256ll + threadIdx.x;
   if (i >= n) return;
   dz[i] = bf(y[i]) > 0.0f ? dy[i] : (uint16_t)0;
-}
-
-// per-channel column sums of a (rows x C) bf16 matrix: partials per block
-__global__ void k_colsum(const uint16_t* __restrict__ a, float* __restrict__ part,
-                         long long rows, int C, long long rows_per_block) {
-  const long long r0 = blockIdx.x * rows_per_block;
-  const long long r1 = r0 + rows_per_block < rows ? r0 + rows_per_block : rows;
-  for (int c = threadIdx.x; c < C; c += 256) {
-    float s = 0.0f;
-    for (long long r = r0; r < r1; ++r) s += bf(a[r * C + c]);
-    part[(long long)blockIdx.x * C + c] = s;
-  }
 }
 
 __global__ void k_avgpool2(const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
@@ -550,25 +459,6 @@ __global__ void k_head(const uint16_t* __restrict__ x, const float* __restrict__
   for (int c = 0; c < C; ++c) s += bf(x[p * C + c]) * w[c];
   const float v = s + bias[0];
   out[p] = scal ? v * scal[0] : v;
-}
-
-// head backward: dx[p][c] = dout[p] w[c]; per-block partials of
-// dw[c] = sum_p dout[p] x[p][c] and db = sum_p dout[p] in part[blk][C+1]
-__global__ void k_head_bwd(const uint16_t* __restrict__ x, const float* __restrict__ w,
-                           const float* __restrict__ dout, uint16_t* __restrict__ dx,
-                           float* __restrict__ part, long long P, int C,
-                           long long rows_per_block) {
-  const long long r0 = blockIdx.x * rows_per_block;
-  const long long r1 = r0 + rows_per_block < P ? r0 + rows_per_block : P;
-  for (long long i = r0 * C + threadIdx.x; i < r1 * C; i += 256) {
-    const long long p = i / C;
-    dx[i] = tobf(dout[p] * w[i % C]);
-  }
-  for (int c = threadIdx.x; c <= C; c += 256) {
-    float s = 0.0f;
-    for (long long p = r0; p < r1; ++p) s += c < C ? dout[p] * bf(x[p * C + c]) : dout[p];
-    part[(long long)blockIdx.x * (C + 1) + c] = s;
-  }
 }
 
 inline unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
@@ -720,41 +610,9 @@ int nx_conv3x3_dgrad(const void* dy, const void* w, void* dx, void* wt, int n, i
   return nx_conv3x3_fwd(dy, wt, nullptr, dx, n, h, wd, cout, cin, 0, stream);
 }
 
-// dw: float32 [cout][9][cin]; work: float32, splits * cout * 9 * cin
-int nx_conv3x3_wgrad(const void* x, const void* dy, float* dw, float* work, int splits,
-                     int n, int h, int wd, int cin, int cout, void* stream) {
-  if (!x || !dy || !dw || !work || splits < 1 || cin % 8 || cout % 8)
-    return nx::set_error(NX_ERR_ARG, "conv3x3 wgrad: cin % 8 == 0 and cout % 8 == 0");
-  const long long M = (long long)n * h * wd;
-  long long per = (M + splits - 1) / splits;
-  per = (per + WG_CHUNK - 1) / WG_CHUNK * WG_CHUNK;
-  const int used = (int)((M + per - 1) / per);
-  const hipStream_t s = NX_U(stream);
-  dim3 grid(((cout + 63) / 64) * ((cin + 63) / 64), 9, used);
-  k_conv3x3_wgrad<<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)dy, work, n,
-                                       h, wd, cin, cout, per);
-  if (hipGetLastError() != hipSuccess) return nx::set_error(NX_ERR_HIP, "wgrad failed");
-  const long long nw = (long long)cout * 9 * cin;
-  k_sum_splits<<<blocks_for(nw), 256, 0, s>>>(work, dw, nw, used);
-  NX_UNET_RET();
-}
-
 int nx_relu_bwd(const void* y, const void* dy, void* dz, long long count, void* stream) {
   k_relu_bwd<<<blocks_for(count), 256, 0, NX_U(stream)>>>(
       (const uint16_t*)y, (const uint16_t*)dy, (uint16_t*)dz, count);
-  NX_UNET_RET();
-}
-
-// column sums of a bf16 (rows x c) matrix into out[c] (float32);
-// work: float32 of blocks * c, blocks = min(1024, rows)
-int nx_colsum(const void* a, float* out, float* work, long long rows, int c,
-              void* stream) {
-  const long long blocks = rows < 1024 ? rows : 1024;
-  const long long per = (rows + blocks - 1) / blocks;
-  const hipStream_t s = NX_U(stream);
-  k_colsum<<<(unsigned)blocks, 256, 0, s>>>((const uint16_t*)a, work, rows, c, per);
-  if (hipGetLastError() != hipSuccess) return nx::set_error(NX_ERR_HIP, "colsum failed");
-  k_sum_splits<<<blocks_for(c), 256, 0, s>>>(work, out, c, (int)blocks);
   NX_UNET_RET();
 }
 
@@ -793,19 +651,6 @@ int nx_head_fwd(const void* x, const float* w, const float* bias, float* out,
                 long long pixels, int c, void* stream) {
   k_head<<<blocks_for(pixels), 256, 0, NX_U(stream)>>>((const uint16_t*)x, w, bias, out,
                                                       pixels, c);
-  NX_UNET_RET();
-}
-
-// dw[c] (c floats) and db (1 float) into dwb[0..c]; work: 1024 * (c+1) floats
-int nx_head_bwd(const void* x, const float* w, const float* dout, void* dx, float* dwb,
-                float* work, long long pixels, int c, void* stream) {
-  const long long blocks = pixels < 1024 ? pixels : 1024;
-  const long long per = (pixels + blocks - 1) / blocks;
-  const hipStream_t s = NX_U(stream);
-  k_head_bwd<<<(unsigned)blocks, 256, 0, s>>>((const uint16_t*)x, w, dout, (uint16_t*)dx,
-                                              work, pixels, c, per);
-  if (hipGetLastError() != hipSuccess) return nx::set_error(NX_ERR_HIP, "head bwd failed");
-  k_sum_splits<<<blocks_for(c + 1), 256, 0, s>>>(work, dwb, c + 1, (int)blocks);
   NX_UNET_RET();
 }
 
