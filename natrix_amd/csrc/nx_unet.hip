@@ -25,6 +25,7 @@
 
 #include "../../include/natrix.h"
 #include "nx_common.h"
+#include "nx_conv.h"
 
 namespace {
 
@@ -495,6 +496,11 @@ static int conv_fwd(const void* x, const void* w, const float* bias, void* y, in
   const uint16_t* ws = (const uint16_t*)w;
   uint16_t* ys = (uint16_t*)y;
   const uint16_t* x2s = (const uint16_t*)x2;
+  if (!part && !tiled && !x2s && !ypool) {
+    hipError_t e;
+    if (nx::conv3x3_lds(xs, ws, bias, ys, n, h, wd, cin, cout, relu, s, &e))
+      return e == hipSuccess ? 0 : nx::set_error(NX_ERR_HIP, hipGetErrorString(e));
+  }
   if (part && used <= KS_WAVES && per <= KS_MAX * KS_PHASES) {
     // every split fits one wave of a workgroup: in-workgroup split-K, one
     // load phase when the splits take at most KS_MAX steps (fewer
@@ -584,7 +590,8 @@ int nx_conv3x3_fwd(const void* x, const void* w, const float* bias, void* y, int
                    int h, int wd, int cin, int cout, int relu, void* stream) {
   if (!x || !w || !y || n < 1 || h < 1 || wd < 1 || cin < 8 || cin % 8 || cout % 32)
     return nx::set_error(NX_ERR_ARG, "conv3x3: channels must be cin % 8 == 0, cout % 32 == 0");
-  conv_fwd(x, w, bias, y, n, h, wd, cin, cout, relu, nullptr, 1, NX_U(stream));
+  const int rc = conv_fwd(x, w, bias, y, n, h, wd, cin, cout, relu, nullptr, 1, NX_U(stream));
+  if (rc != 0) return rc;
   NX_UNET_RET();
 }
 
