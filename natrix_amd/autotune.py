@@ -29,8 +29,9 @@ ARCH = "gfx950"
 
 # (rows, waves, cols) instantiated in csrc/nx_jacobi.hip (NX_TB_SHAPES)
 SHAPES = [(4, 8, 1), (4, 16, 1), (8, 8, 1), (8, 16, 1), (16, 8, 1), (2, 8, 2), (2, 16, 2),
-          (4, 4, 2), (4, 8, 2), (4, 16, 2), (8, 4, 2), (8, 8, 2)]
-KS = (2, 4, 6, 8, 10, 12, 16)
+          (4, 4, 2), (4, 8, 2), (4, 16, 2), (8, 4, 2), (8, 8, 2), (8, 16, 2), (16, 4, 1),
+          (16, 4, 2), (16, 8, 2)]
+KS = (2, 4, 6, 8, 10, 12, 14, 16, 20, 24, 28)
 DEFAULT = (6, 4, 8, 2)
 
 
@@ -52,25 +53,29 @@ def _load():
 
 
 def lookup(W, H, dtype="f32"):
-    """Tuned tile for a W x H grid with `dtype` storage: the exact entry of
-    that storage, else the exact float32 entry, else the float32 entry with
-    the nearest cell count, else the built-in default."""
+    """Tuned tile for a W x H grid with `dtype` storage: the entry of that
+    storage for the grid, else the one with the nearest cell count, else (a
+    storage without entries) the float32 one, else the built-in default.
+    Reduced storage has its own entries because its sweeps per launch are part
+    of its result: the pressure is rounded to storage after every launch, so
+    they stay what they were (12 to 256^2, 16 at 512^2, 10 beyond) and only the
+    tile's shape is tuned."""
     data = _load().get(ARCH, {})
-    key = f"{W}x{H}"
-    if key in data.get(dtype, {}):
-        return tuple(data[dtype][key]["tile"])
-    table = data.get("f32", {})
-    if key in table:
-        return tuple(table[key]["tile"])
-    best, dist = None, None
-    for k, v in table.items():
-        if k.startswith("batch"):
-            continue
-        w, h = (int(t) for t in k.split("x"))
-        d = abs((w * h) - W * H)
-        if dist is None or d < dist:
-            best, dist = tuple(v["tile"]), d
-    return best if best is not None else DEFAULT
+    for table in (data.get(dtype, {}), data.get("f32", {})):
+        key = f"{W}x{H}"
+        if key in table:
+            return tuple(table[key]["tile"])
+        best, dist = None, None
+        for k, v in table.items():
+            if k.startswith("batch"):
+                continue
+            w, h = (int(t) for t in k.split("x"))
+            d = abs((w * h) - W * H)
+            if dist is None or d < dist:
+                best, dist = tuple(v["tile"]), d
+        if best is not None:
+            return best
+    return DEFAULT
 
 
 SMOOTHER_DEFAULT = (8, 4, 8, 2)

@@ -95,8 +95,11 @@ static void invalidate_graphs(nx_sim* s) {
   }
 }
 
-// `sweeps` temporal-blocked sweeps starting from p[pcur]
+// `sweeps` temporal-blocked sweeps starting from p[pcur], in as many launches
+// as c.k sweeps each take, of equal length: the halo a launch recomputes grows
+// with its sweeps, so 25 + 24 costs less than 28 + 21
 int nx::run_jacobi_tb(nx_sim* s, int sweeps, JacobiCfg c) {
+  c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;

@@ -154,12 +154,9 @@ __global__ void __launch_bounds__(WAVES * 64)
     const int s = find_scene(prefix, S, vb);
     const SceneDev d = sc[s];
     const int lb = vb - prefix[s];
-    const int VX = 64 * COLS - 2 * k;
-    const int nbx = (d.W + VX - 1) / VX;
-    jt::jacobi_tb_tile<ROWS, WAVES, COLS>(lb % nbx, lb / nbx, pin + d.off,
-                                          b + d.off, mask + d.off,
-                                          pout + d.off, d.W, d.H, k, nullptr,
-                                          0);
+    const int nx = jt::axis_tiles(d.W, 64 * COLS, k), ny = jt::axis_tiles(d.H, ROWS * WAVES, k);
+    jt::jacobi_tb_tile<ROWS, WAVES, COLS>(lb % nx, lb / nx, nx, ny, pin + d.off, b + d.off,
+                                          mask + d.off, pout + d.off, d.W, d.H, k, nullptr, 0);
     __syncthreads();  // LDS is reused by the next tile
   }
 }
@@ -197,6 +194,7 @@ hipError_t launch_batch_jacobi(const SceneDev* sc, int S, const int* prefix,
     return hipGetLastError();                                                  \
   }
   NX_BJ(4, 8, 1)
+  NX_BJ(4, 16, 1)
   NX_BJ(8, 8, 1)
   NX_BJ(8, 16, 1)
   NX_BJ(16, 8, 1)
@@ -207,6 +205,10 @@ hipError_t launch_batch_jacobi(const SceneDev* sc, int S, const int* prefix,
   NX_BJ(4, 16, 2)
   NX_BJ(8, 4, 2)
   NX_BJ(8, 8, 2)
+  NX_BJ(8, 16, 2)
+  NX_BJ(16, 4, 1)
+  NX_BJ(16, 4, 2)
+  NX_BJ(16, 8, 2)
 #undef NX_BJ
   return hipErrorInvalidValue;
 }
@@ -249,7 +251,7 @@ struct nx_batch {
   std::vector<Splat> splats;  // sorted by scene
   Splat* d_splats = nullptr;
   size_t splat_cap = 0;
-  // prefix tables: key = tile width * 100000 + tile height
+  // prefix tables by tile width and height and sweeps (get_prefix)
   std::map<long long, std::pair<int*, int>> prefix;
   nx_params prm;
   bool timing = false;
@@ -262,8 +264,10 @@ struct nx_batch {
 
 extern "C" int nx_batch_destroy(nx_batch* b);
 
-static int get_prefix(nx_batch* b, int tw, int th, int** dptr, int* total) {
-  const long long key = (long long)tw * 100000 + th;
+// block prefixes of the scenes in tiles of tw x th cells; k: the sweeps whose
+// halo the tiles share (0: none)
+static int get_prefix(nx_batch* b, int tw, int th, int k, int** dptr, int* total) {
+  const long long key = ((long long)tw * 100000 + th) * 256 + k;
   auto it = b->prefix.find(key);
   if (it != b->prefix.end()) {
     *dptr = it->second.first;
@@ -272,7 +276,8 @@ static int get_prefix(nx_batch* b, int tw, int th, int** dptr, int* total) {
   }
   std::vector<int> pre(b->S + 1, 0);
   for (int s = 0; s < b->S; ++s) {
-    const long long n = (long long)((b->W[s] + tw - 1) / tw) * ((b->H[s] + th - 1) / th);
+    const long long n =
+        (long long)jt::axis_tiles(b->W[s], tw, k) * jt::axis_tiles(b->H[s], th, k);
     if (pre[s] + n > (1ll << 30)) return bfail(NX_ERR_ARG, "batch too large");
     pre[s + 1] = pre[s] + (int)n;
   }
@@ -345,13 +350,13 @@ struct BTime {
   } while (0)
 
 static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c) {
+  c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;
     int* pre;
     int total;
-    NXB_TRY(get_prefix(b, 64 * cc.cols - 2 * cc.k, cc.rows * cc.waves - 2 * cc.k,
-                       &pre, &total));
+    NXB_TRY(get_prefix(b, 64 * cc.cols, cc.rows * cc.waves, cc.k, &pre, &total));
     NXB_TIMED(b, NX_TIME_JACOBI,
               launch_batch_jacobi(b->d_scenes, b->S, pre, total, b->p[b->pcur],
                                   b->div, b->mask[b->mcur], b->p[1 - b->pcur], cc,
@@ -366,8 +371,8 @@ static int batch_step(nx_batch* b, float dt) {
   const nx_params& P = b->prm;
   int *pc, *pf;
   int tc, tf;
-  NXB_TRY(get_prefix(b, 64, 4, &pc, &tc));
-  NXB_TRY(get_prefix(b, fused::TX, fused::TY, &pf, &tf));
+  NXB_TRY(get_prefix(b, 64, 4, 0, &pc, &tc));
+  NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &pf, &tf));
   const int a = b->vcur;
   float* dq = b->dye[0] ? b->dye[b->dcur] : nullptr;
   if (!b->splats.empty())
@@ -590,12 +595,13 @@ int nx_batch_update(nx_batch* b, float dt) {
     // make every prefix table exist before capture (no allocation inside)
     int* tmp;
     int tot;
-    NXB_TRY(get_prefix(b, 64, 4, &tmp, &tot));
-    NXB_TRY(get_prefix(b, fused::TX, fused::TY, &tmp, &tot));
+    NXB_TRY(get_prefix(b, 64, 4, 0, &tmp, &tot));
+    NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &tmp, &tot));
     JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols};
-    NXB_TRY(get_prefix(b, 64 * c.cols - 2 * c.k, c.rows * c.waves - 2 * c.k, &tmp, &tot));
+    c.k = jacobi_even_k(P.iterations - 1, c.k);
+    NXB_TRY(get_prefix(b, 64 * c.cols, c.rows * c.waves, c.k, &tmp, &tot));
     const int rem = (P.iterations - 1) % c.k;
-    if (rem) NXB_TRY(get_prefix(b, 64 * c.cols - 2 * rem, c.rows * c.waves - 2 * rem, &tmp, &tot));
+    if (rem) NXB_TRY(get_prefix(b, 64 * c.cols, c.rows * c.waves, rem, &tmp, &tot));
     hipGraph_t g;
     NXB_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     const int vc = b->vcur, mc = b->mcur, dc = b->dcur, pc = b->pcur;

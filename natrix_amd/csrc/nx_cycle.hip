@@ -926,7 +926,7 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
   // a launch with fewer passes has a wider interior, so no launch of the
   // run has more workgroups than one with c.k passes
   const size_t red_need =
-      (size_t)(stream ? stream_launch_blocks(s->W, s->H, c) : jacobi_launch_blocks(s->W, s->H, c)) * 5;
+      (size_t)(stream ? stream_launch_blocks(s->W, s->H, c) : cheb_launch_blocks(s->W, s->H, c)) * 5;
   if (red_need > s->cheb_red_cap) {
     if (s->cheb_red) NX_HIP(hipFree(s->cheb_red));
     s->cheb_red = nullptr;
@@ -963,7 +963,7 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
                                      pending && setup ? s->line : nullptr));
     if (last)
       last_blocks = stream ? stream_launch_blocks(s->W, s->H, cc)
-                           : jacobi_launch_blocks(s->W, s->H, cc);
+                           : cheb_launch_blocks(s->W, s->H, cc);
     s->pcur ^= 1;
     cur ^= 1;
     done += its;

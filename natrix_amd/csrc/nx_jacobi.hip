@@ -2,23 +2,28 @@
 //
 // One launch performs k consecutive sweeps of shader.Poisson.comp:24-37 on a
 // tile held in registers.  A block is WAVES wavefronts stacked vertically;
-// each lane owns one x column and ROWS consecutive rows of it, so:
+// each lane owns COLS adjacent x columns and ROWS consecutive rows of them, so:
 //   * vertical neighbours inside a lane's strip are registers,
-//   * horizontal neighbours are the adjacent lanes' registers, read with the
+//   * horizontal neighbours are registers or the adjacent lanes', read with the
 //     DPP wave_shr:1 / wave_shl:1 lane shifts (no LDS traffic),
 //   * the rows just above/below a wave's strip come from the neighbouring
 //     wave through a small double-buffered LDS exchange (one barrier/sweep).
-// The block reads a (64) x (ROWS*WAVES) tile once, sweeps k times, and writes
-// back the (64-2k) x (ROWS*WAVES-2k) interior whose k-step dependency cone
-// stayed inside the tile.  Each sweep evaluates exactly the reference's
-// expression for every cell, so k sweeps per launch are bitwise equal to k
-// single sweeps.
+// The block reads its tile once, sweeps k times, and writes back the cells
+// whose k-step dependency cone stayed inside the tile (nx_jacobi_tile.h: the
+// tiling).  Each sweep evaluates exactly the reference's expression for every
+// cell, so k sweeps per launch are bitwise equal to k single sweeps.
 //
-// Out-of-grid tile cells and the reference's clamp-to-edge neighbours
-// (common.sh:14-17) are both expressed as "use the centre value", which is
-// also what a solid neighbour does (Poisson.comp:32-35): a 4-bit code per
-// cell says which neighbours are replaced (bit 4: the cell is not fluid).  Wavefronts whose codes are all
-// zero (the bulk of the grid) take a select-free path.
+// The reference's clamp-to-edge neighbours (common.sh:14-17) and solid
+// neighbours (Poisson.comp:32-35) are both "use the centre value".  A wave
+// takes the sweep's select-free form when its strip touches neither.
+//
+// Bound: with many tiles, VALU issue (a wave64 addition takes 2 cycles when
+// two waves or more share a SIMD, a DPP one 4: 12 cycles per pair of columns
+// and row) and, between blocks, the load of the next tile; with few, the
+// exchange's latency.  Per sweep, launch gaps included: 2048^2 (13, 8, 8, 2)
+// 1.97 us (2.99 before the in-grid tiles, masks on demand and the register
+// walk, with tile (10, 8, 8, 1)), 4096^2 (20, 16, 8, 2) 5.4 us (8.76), 1024^2
+// (20, 4, 16, 2) 1.07 us (1.48), 256^2 (24, 4, 16, 1) 0.48 us (0.69).
 #include "nx_jacobi_tile.h"
 #include "nx_kernels.h"
 
@@ -28,21 +33,19 @@ namespace {
 
 using jt::wave_sum;
 
-template <int ROWS, int WAVES, int COLS>
+template <int ROWS, int WAVES, int COLS, bool RES>
 __global__ void __launch_bounds__(WAVES * 64)
     __attribute__((amdgpu_waves_per_eu(jt::jacobi_waves_per_eu<ROWS * COLS>())))
     k_jacobi_tb(const float* __restrict__ pin, const float* __restrict__ b,
                 const uint8_t* __restrict__ mask, float* __restrict__ pout,
-                int W, int H, int k, double* __restrict__ red,
+                int W, int H, int k, int nx, int ny, double* __restrict__ red,
                 const int* __restrict__ done) {
   if (done != nullptr && *done != 0) return;  // block-uniform early exit
-  // 1D grid of gx * gy tiles in XCD order; the partial-sum record is the
+  // 1D grid of nx * ny tiles in XCD order; the partial-sum record is the
   // tile's row-major index
-  const int gx = (W + 64 * COLS - 2 * k - 1) / (64 * COLS - 2 * k);
-  const int gy = (H + ROWS * WAVES - 2 * k - 1) / (ROWS * WAVES - 2 * k);
-  const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, gx * gy);
-  jt::jacobi_tb_tile<ROWS, WAVES, COLS>(t % gx, t / gx, pin, b, mask, pout, W, H, k, red,
-                                        t);
+  const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, nx * ny);
+  jt::jacobi_tb_tile<ROWS, WAVES, COLS, F32S, false, RES>(t % nx, t / nx, nx, ny, pin, b, mask,
+                                                          pout, W, H, k, red, t);
 }
 
 // Exact FP64 residual of p (or of a zero guess when p == nullptr) plus the
@@ -175,11 +178,13 @@ template <int ROWS, int WAVES, int COLS>
 hipError_t launch_tb(const float* pin, const float* b, const uint8_t* mask,
                      float* pout, int W, int H, int k, double* red,
                      const int* done, hipStream_t s) {
-  constexpr int EX = 64 * COLS, EY = ROWS * WAVES;
-  const int VX = EX - 2 * k, VY = EY - 2 * k;
-  const dim3 grid(((W + VX - 1) / VX) * ((H + VY - 1) / VY), 1, 1);
-  k_jacobi_tb<ROWS, WAVES, COLS><<<grid, WAVES * 64, 0, s>>>(
-      pin, b, mask, pout, W, H, k, red, done);
+  const int nx = jt::axis_tiles(W, 64 * COLS, k), ny = jt::axis_tiles(H, ROWS * WAVES, k);
+  if (red)
+    k_jacobi_tb<ROWS, WAVES, COLS, true><<<nx * ny, WAVES * 64, 0, s>>>(
+        pin, b, mask, pout, W, H, k, nx, ny, red, done);
+  else
+    k_jacobi_tb<ROWS, WAVES, COLS, false><<<nx * ny, WAVES * 64, 0, s>>>(
+        pin, b, mask, pout, W, H, k, nx, ny, red, done);
   return hipGetLastError();
 }
 
@@ -199,7 +204,11 @@ hipError_t launch_tb(const float* pin, const float* b, const uint8_t* mask,
   X(4, 8, 2)            \
   X(4, 16, 2)           \
   X(8, 4, 2)            \
-  X(8, 8, 2)
+  X(8, 8, 2)            \
+  X(8, 16, 2)           \
+  X(16, 4, 1)           \
+  X(16, 4, 2)           \
+  X(16, 8, 2)
 
 bool jacobi_cfg_supported(JacobiCfg c) {
   if (c.seg != 0) return c.seg > 0 && stream_cfg_supported(c);
@@ -215,6 +224,10 @@ bool jacobi_cfg_supported(JacobiCfg c) {
 
 int jacobi_launch_blocks(int W, int H, JacobiCfg c) {
   if (c.seg > 0) return stream_launch_blocks(W, H, c);
+  return jt::axis_tiles(W, 64 * c.cols, c.k) * jt::axis_tiles(H, c.rows * c.waves, c.k);
+}
+
+int cheb_launch_blocks(int W, int H, JacobiCfg c) {
   const int VX = 64 * c.cols - 2 * c.k, VY = c.rows * c.waves - 2 * c.k;
   return ((W + VX - 1) / VX) * ((H + VY - 1) / VY);
 }

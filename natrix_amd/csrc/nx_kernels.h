@@ -75,7 +75,15 @@ struct JacobiCfg {
   int cols;     // columns per lane
   int seg = 0;  // > 0: streaming kernel, output rows per workgroup segment
 };
+// sweeps per launch that spread `sweeps` evenly over ceil(sweeps / k) launches
+inline int jacobi_even_k(int sweeps, int k) {
+  if (sweeps <= 0) return k;
+  const int n = (sweeps + k - 1) / k;
+  return (sweeps + n - 1) / n;
+}
 int jacobi_launch_blocks(int W, int H, JacobiCfg cfg);
+// workgroups of a fine Chebyshev tile launch
+int cheb_launch_blocks(int W, int H, JacobiCfg cfg);
 hipError_t launch_jacobi_tb(const float* pin, const float* b,
                             const uint8_t* mask, float* pout, int W, int H,
                             JacobiCfg cfg, double* red, const int* done,
@@ -113,7 +121,7 @@ int smooth_chebyshev_pending(::nx_sim* s, int iterations, float lambda_min, cons
 // red, the last pass instead evaluates the exact FP64 residual b - L x of
 // the final iterate on the written interior and each block writes
 // red[5 blk + {sum r, sum r^2, sum b, sum b^2, fluid cells}] (blocks:
-// jacobi_launch_blocks of the launch's shape and passes).  With dapp (first
+// cheb_launch_blocks of the launch's shape and passes).  With dapp (first
 // launch), the loaded x first takes a pending line-search step: x += a dapp
 // on fluid cells, a = (float)line[0], nothing when a == 0.
 constexpr int CHEB_MAX_PASSES = 32;

@@ -52,13 +52,11 @@ __global__ void __launch_bounds__(WAVES * 64)
     km_jacobi(const typename S::s1* __restrict__ pin,
               const typename S::s1* __restrict__ b,
               const uint8_t* __restrict__ mask, typename S::s1* __restrict__ pout,
-              float* __restrict__ pout32, int W, int H, int k) {
-  // 1D grid of gx * gy tiles in XCD order
-  const int gx = (W + 64 * COLS - 2 * k - 1) / (64 * COLS - 2 * k);
-  const int gy = (H + ROWS * WAVES - 2 * k - 1) / (ROWS * WAVES - 2 * k);
-  const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, gx * gy);
-  jt::jacobi_tb_tile<ROWS, WAVES, COLS, S, CORR>(t % gx, t / gx, pin, b, mask, pout, W, H,
-                                                 k, nullptr, 0, pout32);
+              float* __restrict__ pout32, int W, int H, int k, int nx, int ny) {
+  // 1D grid of nx * ny tiles in XCD order
+  const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, nx * ny);
+  jt::jacobi_tb_tile<ROWS, WAVES, COLS, S, CORR>(t % nx, t / nx, nx, ny, pin, b, mask, pout, W,
+                                                 H, k, nullptr, 0, pout32);
 }
 
 template <class S>
@@ -127,17 +125,16 @@ template <int R, int WV, int CL, class S>
 hipError_t mixed_tb(const void* pin, const void* b, const uint8_t* mask,
                     void* pout, float* pout32, int W, int H, int k, bool corr,
                     hipStream_t s) {
-  constexpr int EX = 64 * CL, EY = R * WV;
-  const dim3 grid(((W + EX - 2 * k - 1) / (EX - 2 * k)) * ((H + EY - 2 * k - 1) / (EY - 2 * k)),
-                  1, 1);
+  const int nx = jt::axis_tiles(W, 64 * CL, k), ny = jt::axis_tiles(H, R * WV, k);
+  const dim3 grid(nx * ny);
   if (corr)
     km_jacobi<R, WV, CL, S, true><<<grid, WV * 64, 0, s>>>(
         (const typename S::s1*)pin, (const typename S::s1*)b, mask,
-        (typename S::s1*)pout, pout32, W, H, k);
+        (typename S::s1*)pout, pout32, W, H, k, nx, ny);
   else
     km_jacobi<R, WV, CL, S, false><<<grid, WV * 64, 0, s>>>(
         (const typename S::s1*)pin, (const typename S::s1*)b, mask,
-        (typename S::s1*)pout, pout32, W, H, k);
+        (typename S::s1*)pout, pout32, W, H, k, nx, ny);
   return hipGetLastError();
 }
 
@@ -149,6 +146,7 @@ hipError_t mixed_tb_shape(const void* pin, const void* b, const uint8_t* mask,
   if (c.rows == R && c.waves == WV && c.cols == CL)                       \
     return mixed_tb<R, WV, CL, S>(pin, b, mask, pout, pout32, W, H, c.k, corr, s);
   NX_MTB(4, 8, 1)
+  NX_MTB(4, 16, 1)
   NX_MTB(8, 8, 1)
   NX_MTB(8, 16, 1)
   NX_MTB(16, 8, 1)
@@ -159,6 +157,10 @@ hipError_t mixed_tb_shape(const void* pin, const void* b, const uint8_t* mask,
   NX_MTB(4, 16, 2)
   NX_MTB(8, 4, 2)
   NX_MTB(8, 8, 2)
+  NX_MTB(8, 16, 2)
+  NX_MTB(16, 4, 1)
+  NX_MTB(16, 4, 2)
+  NX_MTB(16, 8, 2)
 #undef NX_MTB
   return hipErrorInvalidValue;
 }
