@@ -97,16 +97,23 @@ static void invalidate_graphs(nx_sim* s) {
 
 // `sweeps` temporal-blocked sweeps starting from p[pcur], in as many launches
 // as c.k sweeps each take, of equal length: the halo a launch recomputes grows
-// with its sweeps, so 25 + 24 costs less than 28 + 21
-int nx::run_jacobi_tb(nx_sim* s, int sweeps, JacobiCfg c) {
+// with its sweeps, so 25 + 24 costs less than 28 + 21.  u != nullptr (tile
+// shapes): the last launch projects u in place and writes the next step's mask.
+int nx::run_jacobi_tb(nx_sim* s, int sweeps, JacobiCfg c, float2* u) {
   c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;
-    NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
-                    launch_jacobi_tb(s->p[s->pcur], s->div, s->mask[s->mcur],
-                                     s->p[1 - s->pcur], s->W, s->H, cc,
-                                     nullptr, nullptr, s->stream));
+    if (u && sweeps == cc.k)
+      NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
+                      launch_jacobi_project(s->p[s->pcur], s->div, s->mask[s->mcur],
+                                            s->p[1 - s->pcur], u, s->mask[1 - s->mcur], s->W,
+                                            s->H, cc, s->stream));
+    else
+      NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
+                      launch_jacobi_tb(s->p[s->pcur], s->div, s->mask[s->mcur],
+                                       s->p[1 - s->pcur], s->W, s->H, cc,
+                                       nullptr, nullptr, s->stream));
     s->pcur ^= 1;
     sweeps -= cc.k;
   }
@@ -286,29 +293,55 @@ static int step_reference_order(nx_sim* s, float dt) {
   return NX_OK;
 }
 
-// Fused step: advect (walls folded into its reads), fused curl..p1,
-// temporal-blocked Jacobi, projection + obstacle clear, dye advection.
+// The fused step has two forms with the same results.  Merged: the advection
+// runs in the kernel of the following stages (each tile advects its halo's
+// cells once more, 1.5 times the gathers, which stay in the caches, instead of
+// writing and reading the advected velocity) and the projection in the last
+// Jacobi (or correction) launch, in place, with the pressure it holds: two
+// launches and 21 bytes a cell less.  Separate: one launch per family, where
+// the families are timed one by one, where the streaming kernel sweeps, and
+// where the pressure is not made by a plain sequence of sweeps.
+static bool step_merged(const nx_sim* s, bool tolerance) {
+  return !s->timing && !tolerance &&
+         (s->storage != ST_F32 || (s->prm.iterations > 1 && s->prm.jacobi_seg == 0));
+}
+
+static void viscosity_of(const nx_params& P, int& viscous, float& alpha, float& rbeta) {
+  viscous = P.viscosity > 0.0f;
+  alpha = rbeta = 0.0f;
+  if (viscous) {
+    const double av = 1.0 / (double)P.viscosity;
+    alpha = (float)av;
+    rbeta = (float)(1.0 / (4.0 + av));
+  }
+}
+
 // Reduced-precision step: the fused sequence with every field stored in
 // bfloat16/float16, then the float32 residual-correction launch.
 static int step_mixed_enqueue(nx_sim* s, float dt) {
   const nx_params& P = s->prm;
   const int W = s->W, H = s->H, st = s->storage;
   const int a = s->vcur;
-  NX_LAUNCH_TIMED(s, NX_TIME_ADVECT,
-                  launch_m_advect(st, s->vel[a], s->vel[1 - a], s->mask[s->mcur],
-                                  W, H, dt, P.speed, P.dissipation, bc_of(P),
-                                  s->stream));
-  float alpha = 0.0f, rbeta = 0.0f;
-  const int viscous = P.viscosity > 0.0f;
-  if (viscous) {
-    const double av = 1.0 / (double)P.viscosity;
-    alpha = (float)av;
-    rbeta = (float)(1.0 / (4.0 + av));
+  const bool merged = step_merged(s, false);
+  float alpha, rbeta;
+  int viscous;
+  viscosity_of(P, viscous, alpha, rbeta);
+  if (merged) {
+    NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
+                    launch_m_advect_fused(st, s->vel[a], s->mask[s->mcur], s->vel[1 - a],
+                                          s->div, s->p[0], W, H, dt, P.speed, P.dissipation,
+                                          bc_of(P), P.vorticity, viscous, alpha, rbeta,
+                                          s->stream));
+  } else {
+    NX_LAUNCH_TIMED(s, NX_TIME_ADVECT,
+                    launch_m_advect(st, s->vel[a], s->vel[1 - a], s->mask[s->mcur],
+                                    W, H, dt, P.speed, P.dissipation, bc_of(P),
+                                    s->stream));
+    NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
+                    launch_m_fused(st, s->vel[1 - a], s->mask[s->mcur], s->vel[a],
+                                   s->div, s->p[0], W, H, dt, P.vorticity, viscous,
+                                   alpha, rbeta, s->stream));
   }
-  NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
-                  launch_m_fused(st, s->vel[1 - a], s->mask[s->mcur], s->vel[a],
-                                 s->div, s->p[0], W, H, dt, P.vorticity, viscous,
-                                 alpha, rbeta, s->stream));
   s->pcur = 0;
   JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols, P.jacobi_seg};
   int sweeps = P.iterations - 1;
@@ -326,15 +359,22 @@ static int step_mixed_enqueue(nx_sim* s, float dt) {
   // sweeps of A e = r, written as p + e (with 0 sweeps: the widened p)
   JacobiCfg cr = c;
   cr.k = 1 + P.correction_sweeps;
-  NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
-                  launch_m_jacobi(st, s->p[s->pcur], s->div, s->mask[s->mcur],
-                                  nullptr, s->p32, W, H, cr, true, s->stream));
+  if (merged) {
+    NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
+                    launch_m_correct_project(st, s->p[s->pcur], s->div, s->mask[s->mcur],
+                                             s->p32, s->vel[1 - a], s->mask[1 - s->mcur], W, H,
+                                             cr, s->stream));
+  } else {
+    NX_LAUNCH_TIMED(s, NX_TIME_JACOBI,
+                    launch_m_jacobi(st, s->p[s->pcur], s->div, s->mask[s->mcur],
+                                    nullptr, s->p32, W, H, cr, true, s->stream));
+    NX_LAUNCH_TIMED(s, NX_TIME_PROJECT,
+                    launch_m_subgrad(st, s->vel[a], s->p32, s->mask[s->mcur],
+                                     s->vel[1 - a], s->mask[1 - s->mcur], W, H,
+                                     s->stream));
+  }
   s->stats.sweeps = P.iterations;
   s->stats.converged = 0;
-  NX_LAUNCH_TIMED(s, NX_TIME_PROJECT,
-                  launch_m_subgrad(st, s->vel[a], s->p32, s->mask[s->mcur],
-                                   s->vel[1 - a], s->mask[1 - s->mcur], W, H,
-                                   s->stream));
   s->vcur = 1 - a;
   s->mcur ^= 1;
   if (s->dye[0] && P.dye_in_step) {
@@ -353,36 +393,43 @@ static int step_fused_enqueue(nx_sim* s, float dt, bool tolerance) {
   const nx_params& P = s->prm;
   const int W = s->W, H = s->H;
   const int a = s->vcur;
-  NX_LAUNCH_TIMED(s, NX_TIME_ADVECT,
-                  launch_advect(s->vel[a], s->vel[1 - a], s->mask[s->mcur], W,
-                                H, dt, P.speed, P.dissipation, bc_of(P),
-                                s->stream));
-  float alpha = 0.0f, rbeta = 0.0f;
-  const int viscous = P.viscosity > 0.0f;
-  if (viscous) {
-    const double av = 1.0 / (double)P.viscosity;
-    alpha = (float)av;
-    rbeta = (float)(1.0 / (4.0 + av));
-  }
-  NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
-                  launch_fused_vort_div(s->vel[1 - a], s->mask[s->mcur],
-                                        s->vel[a], s->div, s->p[0], W, H, dt,
-                                        P.vorticity, viscous, alpha, rbeta,
-                                        s->stream));
-  s->pcur = 0;
-  if (tolerance) {
-    NX_TRY(solve_tolerance(s, 1, true));
+  const bool merged = step_merged(s, tolerance);
+  float alpha, rbeta;
+  int viscous;
+  viscosity_of(P, viscous, alpha, rbeta);
+  JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols, P.jacobi_seg};
+  if (merged) {
+    NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
+                    launch_advect_vort_div(s->vel[a], s->mask[s->mcur], s->vel[1 - a], s->div,
+                                           s->p[0], W, H, dt, P.speed, P.dissipation, bc_of(P),
+                                           P.vorticity, viscous, alpha, rbeta, s->stream));
+    s->pcur = 0;
+    NX_TRY(run_jacobi_tb(s, P.iterations - 1, c, s->vel[1 - a]));
   } else {
-    JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols, P.jacobi_seg};
-    NX_TRY(run_jacobi_tb(s, P.iterations - 1, c));
+    NX_LAUNCH_TIMED(s, NX_TIME_ADVECT,
+                    launch_advect(s->vel[a], s->vel[1 - a], s->mask[s->mcur], W,
+                                  H, dt, P.speed, P.dissipation, bc_of(P),
+                                  s->stream));
+    NX_LAUNCH_TIMED(s, NX_TIME_VORT_DIV,
+                    launch_fused_vort_div(s->vel[1 - a], s->mask[s->mcur],
+                                          s->vel[a], s->div, s->p[0], W, H, dt,
+                                          P.vorticity, viscous, alpha, rbeta,
+                                          s->stream));
+    s->pcur = 0;
+    if (tolerance)
+      NX_TRY(solve_tolerance(s, 1, true));
+    else
+      NX_TRY(run_jacobi_tb(s, P.iterations - 1, c));
+    NX_LAUNCH_TIMED(s, NX_TIME_PROJECT,
+                    launch_subtract_gradient(s->vel[a], s->p[s->pcur],
+                                             s->mask[s->mcur], s->vel[1 - a],
+                                             s->mask[1 - s->mcur], W, H,
+                                             s->stream));
+  }
+  if (!tolerance) {
     s->stats.sweeps = P.iterations;
     s->stats.converged = 0;
   }
-  NX_LAUNCH_TIMED(s, NX_TIME_PROJECT,
-                  launch_subtract_gradient(s->vel[a], s->p[s->pcur],
-                                           s->mask[s->mcur], s->vel[1 - a],
-                                           s->mask[1 - s->mcur], W, H,
-                                           s->stream));
   s->vcur = 1 - a;
   s->mcur ^= 1;
   if (s->dye[0] && P.dye_in_step) {

@@ -124,6 +124,8 @@ __global__ void __launch_bounds__(256)
 
 #undef NX_BATCH_CELL_LOOP
 
+// ADV: with the advection in front (kb_advect then kb_fused, one pass)
+template <bool ADV>
 __global__ void __launch_bounds__(256)
     kb_fused(const SceneDev* __restrict__ sc, int S,
              const int* __restrict__ prefix, int total,
@@ -135,28 +137,32 @@ __global__ void __launch_bounds__(256)
     const SceneDev d = sc[s];
     const int lb = vb - prefix[s];
     const int nbx = (d.W + fused::TX - 1) / fused::TX;
-    fused::fused_vort_div_tile((lb % nbx) * fused::TX, (lb / nbx) * fused::TY,
-                               uin + d.off, mask + d.off, uout + d.off,
-                               div + d.off, p1 + d.off, d.W, d.H, dt, d.vort,
-                               d.viscous, d.alpha, d.rbeta);
+    fused::fused_vort_div_tile<F32S, ADV>(
+        (lb % nbx) * fused::TX, (lb / nbx) * fused::TY, uin + d.off, mask + d.off, uout + d.off,
+        div + d.off, p1 + d.off, d.W, d.H, dt, d.vort, d.viscous, d.alpha, d.rbeta,
+        fused::Advect{ADV, d.speed, d.diss, d.bc});
     __syncthreads();  // LDS is reused by the next tile
   }
 }
 
-template <int ROWS, int WAVES, int COLS>
+template <int ROWS, int WAVES, int COLS, bool PROJ>
 __global__ void __launch_bounds__(WAVES * 64)
+    __attribute__((amdgpu_waves_per_eu(jt::jacobi_waves_per_eu<ROWS * COLS>())))
     kb_jacobi(const SceneDev* __restrict__ sc, int S,
               const int* __restrict__ prefix, int total,
               const float* __restrict__ pin, const float* __restrict__ b,
               const uint8_t* __restrict__ mask, float* __restrict__ pout,
-              int k) {
+              int k, float2* u, uint8_t* mask_next) {
   for (int vb = blockIdx.x; vb < total; vb += gridDim.x) {
     const int s = find_scene(prefix, S, vb);
     const SceneDev d = sc[s];
     const int lb = vb - prefix[s];
-    const int nx = jt::axis_tiles(d.W, 64 * COLS, k), ny = jt::axis_tiles(d.H, ROWS * WAVES, k);
-    jt::jacobi_tb_tile<ROWS, WAVES, COLS>(lb % nx, lb / nx, nx, ny, pin + d.off, b + d.off,
-                                          mask + d.off, pout + d.off, d.W, d.H, k, nullptr, 0);
+    const int kt = PROJ ? k + 1 : k;
+    const int nx = jt::axis_tiles(d.W, 64 * COLS, kt), ny = jt::axis_tiles(d.H, ROWS * WAVES, kt);
+    jt::jacobi_tb_tile<ROWS, WAVES, COLS, F32S, false, false, PROJ>(
+        lb % nx, lb / nx, nx, ny, pin + d.off, b + d.off, mask + d.off, pout + d.off, d.W, d.H, k,
+        nullptr, 0, nullptr,
+        jt::Project<F32S>{PROJ ? u + d.off : nullptr, PROJ ? mask_next + d.off : nullptr});
     __syncthreads();  // LDS is reused by the next tile
   }
 }
@@ -182,15 +188,22 @@ int resident_grid(K kernel, int block_threads, int total) {
 }  // namespace
 
 // ---- launchers used by the batch object --------------------------------
+// u != nullptr: the projection of u (in place) and the next step's masks too
 hipError_t launch_batch_jacobi(const SceneDev* sc, int S, const int* prefix,
                                int total, const float* pin, const float* b,
-                               const uint8_t* mask, float* pout, JacobiCfg c,
-                               hipStream_t s) {
+                               const uint8_t* mask, float* pout, JacobiCfg c, float2* u,
+                               uint8_t* mask_next, hipStream_t s) {
 #define NX_BJ(R, WV, CL)                                                       \
   if (c.rows == R && c.waves == WV && c.cols == CL) {                          \
-    const int g = resident_grid(kb_jacobi<R, WV, CL>, WV * 64, total);         \
-    kb_jacobi<R, WV, CL><<<g, WV * 64, 0, s>>>(sc, S, prefix, total, pin, b,   \
-                                               mask, pout, c.k);               \
+    if (u) {                                                                   \
+      const int g = resident_grid(kb_jacobi<R, WV, CL, true>, WV * 64, total); \
+      kb_jacobi<R, WV, CL, true><<<g, WV * 64, 0, s>>>(                        \
+          sc, S, prefix, total, pin, b, mask, pout, c.k, u, mask_next);        \
+    } else {                                                                   \
+      const int g = resident_grid(kb_jacobi<R, WV, CL, false>, WV * 64, total); \
+      kb_jacobi<R, WV, CL, false><<<g, WV * 64, 0, s>>>(                       \
+          sc, S, prefix, total, pin, b, mask, pout, c.k, nullptr, nullptr);    \
+    }                                                                          \
     return hipGetLastError();                                                  \
   }
   NX_BJ(4, 8, 1)
@@ -349,20 +362,47 @@ struct BTime {
     t_.end();                                                         \
   } while (0)
 
-static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c) {
+// project: the last launch also projects vel[1 - vcur] and writes the next masks
+static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c, bool project = false) {
   c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;
+    const bool last = project && sweeps == cc.k;
     int* pre;
     int total;
-    NXB_TRY(get_prefix(b, 64 * cc.cols, cc.rows * cc.waves, cc.k, &pre, &total));
+    NXB_TRY(get_prefix(b, 64 * cc.cols, cc.rows * cc.waves, cc.k + (last ? 1 : 0), &pre, &total));
     NXB_TIMED(b, NX_TIME_JACOBI,
               launch_batch_jacobi(b->d_scenes, b->S, pre, total, b->p[b->pcur],
                                   b->div, b->mask[b->mcur], b->p[1 - b->pcur], cc,
+                                  last ? b->vel[1 - b->vcur] : nullptr, b->mask[1 - b->mcur],
                                   b->stream));
     b->pcur ^= 1;
     sweeps -= cc.k;
+  }
+  return NX_OK;
+}
+
+// one launch for the advection and the stages up to the first sweep, and the
+// projection in the last Jacobi launch, unless the kernels are timed one by one
+// or there is no further sweep
+static bool batch_step_merged(const nx_batch* b) { return !b->timing && b->prm.iterations > 1; }
+
+// every prefix table a step needs (no allocation inside a capture)
+static int batch_step_tables(nx_batch* b) {
+  const nx_params& P = b->prm;
+  int* tmp;
+  int tot;
+  NXB_TRY(get_prefix(b, 64, 4, 0, &tmp, &tot));
+  NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &tmp, &tot));
+  int sweeps = P.iterations - 1;
+  const int k = jacobi_even_k(sweeps, P.jacobi_k);
+  while (sweeps > 0) {
+    const int kk = std::min(sweeps, k);
+    const bool last = batch_step_merged(b) && sweeps == kk;
+    NXB_TRY(get_prefix(b, 64 * P.jacobi_cols, P.jacobi_rows * P.jacobi_waves, kk + (last ? 1 : 0),
+                       &tmp, &tot));
+    sweeps -= kk;
   }
   return NX_OK;
 }
@@ -374,20 +414,27 @@ static int batch_step(nx_batch* b, float dt) {
   NXB_TRY(get_prefix(b, 64, 4, 0, &pc, &tc));
   NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &pf, &tf));
   const int a = b->vcur;
+  const bool merged = batch_step_merged(b);
   float* dq = b->dye[0] ? b->dye[b->dcur] : nullptr;
   if (!b->splats.empty())
     NXB_KERNEL(b, NX_TIME_SPLAT, kb_splats, tc, b->d_scenes, b->S, pc, tc,
                b->vel[a], dq, b->d_splats);
-  NXB_KERNEL(b, NX_TIME_ADVECT, kb_advect, tc, b->d_scenes, b->S, pc, tc,
-             b->vel[a], b->vel[1 - a], b->mask[b->mcur], dt);
-  NXB_KERNEL(b, NX_TIME_VORT_DIV, kb_fused, tf, b->d_scenes, b->S, pf, tf,
-             b->vel[1 - a], b->mask[b->mcur], b->vel[a], b->div, b->p[0], dt);
+  if (merged) {
+    NXB_KERNEL(b, NX_TIME_VORT_DIV, kb_fused<true>, tf, b->d_scenes, b->S, pf, tf,
+               b->vel[a], b->mask[b->mcur], b->vel[1 - a], b->div, b->p[0], dt);
+  } else {
+    NXB_KERNEL(b, NX_TIME_ADVECT, kb_advect, tc, b->d_scenes, b->S, pc, tc,
+               b->vel[a], b->vel[1 - a], b->mask[b->mcur], dt);
+    NXB_KERNEL(b, NX_TIME_VORT_DIV, kb_fused<false>, tf, b->d_scenes, b->S, pf, tf,
+               b->vel[1 - a], b->mask[b->mcur], b->vel[a], b->div, b->p[0], dt);
+  }
   b->pcur = 0;
   JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols};
-  NXB_TRY(batch_jacobi(b, P.iterations - 1, c));
-  NXB_KERNEL(b, NX_TIME_PROJECT, kb_subgrad, tc, b->d_scenes, b->S, pc, tc,
-             b->vel[a], b->p[b->pcur], b->mask[b->mcur], b->vel[1 - a],
-             b->mask[1 - b->mcur]);
+  NXB_TRY(batch_jacobi(b, P.iterations - 1, c, merged));
+  if (!merged)
+    NXB_KERNEL(b, NX_TIME_PROJECT, kb_subgrad, tc, b->d_scenes, b->S, pc, tc,
+               b->vel[a], b->p[b->pcur], b->mask[b->mcur], b->vel[1 - a],
+               b->mask[1 - b->mcur]);
   b->vcur = 1 - a;
   b->mcur ^= 1;
   if (b->dye[0]) {
@@ -592,16 +639,7 @@ int nx_batch_update(nx_batch* b, float dt) {
       memcmp(&b->graph_prm[par], &P, sizeof(P)) != 0) {
     if (b->graph[par]) NXB_HIP(hipGraphExecDestroy(b->graph[par]));
     b->graph[par] = nullptr;
-    // make every prefix table exist before capture (no allocation inside)
-    int* tmp;
-    int tot;
-    NXB_TRY(get_prefix(b, 64, 4, 0, &tmp, &tot));
-    NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &tmp, &tot));
-    JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols};
-    c.k = jacobi_even_k(P.iterations - 1, c.k);
-    NXB_TRY(get_prefix(b, 64 * c.cols, c.rows * c.waves, c.k, &tmp, &tot));
-    const int rem = (P.iterations - 1) % c.k;
-    if (rem) NXB_TRY(get_prefix(b, 64 * c.cols, c.rows * c.waves, rem, &tmp, &tot));
+    NXB_TRY(batch_step_tables(b));
     hipGraph_t g;
     NXB_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     const int vc = b->vcur, mc = b->mcur, dc = b->dcur, pc = b->pcur;

@@ -1,6 +1,8 @@
-// Fused curl -> confinement -> [viscosity] -> divergence -> first sweep,
-// one LDS-staged 64x16 tile (shared by the single-grid and batched kernels).
+// Fused [advection ->] curl -> confinement -> [viscosity] -> divergence ->
+// first sweep, one LDS-staged 64x16 tile (shared by the single-grid and batched
+// kernels).
 #pragma once
+#include "nx_cells.h"
 #include "nx_common.h"
 
 namespace nx {
@@ -36,18 +38,26 @@ __device__ __forceinline__ float2 confine_cell(float2 u, float wc, float wl,
   return make_float2(u.x + fx * dt, u.y + fy * dt);
 }
 
+// The advection of the velocity that enters a tile (Advect::on), with the
+// walls' treatment on its reads; off: the input is the advected velocity.
+struct Advect {
+  int on;
+  float speed, diss;
+  BcParams bc;
+};
+
 // Stages of one 64x16 output tile with halo HA (3, or 4 with viscosity);
-// every stage walks its region as one flat index range over the block's 256
+// every stage walks its region as one flat index range over the block's NT
 // threads, so no lane idles on the few columns past a multiple of 64.  In
 // an INTERIOR tile (halo inside the grid) no coordinate clamps, and the
 // stencil neighbours of a stage slot are fixed offsets in the previous
 // stage's array; border tiles evaluate the clamped coordinates.
-template <class S, bool VISC, bool INTERIOR>
+template <class S, bool VISC, bool INTERIOR, bool ADV, int NT>
 __device__ __forceinline__ void fused_tile_stages(
     float2* A, float* Wc, float2* V2, const Tile& t, const typename S::s2* __restrict__ uin,
     const uint8_t* __restrict__ mask, typename S::s2* __restrict__ uout,
     typename S::s1* __restrict__ div, typename S::s1* __restrict__ p1, float dt,
-    float scale, float alpha, float rbeta) {
+    float scale, float alpha, float rbeta, const Advect& adv) {
   constexpr int hA = VISC ? 4 : 3, hW = hA - 1, hV2 = hA - 2;
   constexpr int WA = TX + 2 * hA, HA = TY + 2 * hA;
   constexpr int WW = TX + 2 * hW, HW = TY + 2 * hW;
@@ -58,20 +68,70 @@ __device__ __forceinline__ void fused_tile_stages(
   // confinement stage, which a barrier separates from the viscosity stage
   float2* const V3 = A;
 
-  // 1. advected velocity at clamped coordinates
-  for (int k = tid; k < WA * HA; k += 256) {
+  // 1. advected velocity at clamped coordinates; advected here, the halo's
+  //    cells are advected by every tile that reads them, and rounded to
+  //    storage as a pass of its own would leave them
+  auto slot = [&](int k, int& gx, int& gy) {
     const int j = k / WA, i = k - j * WA;
-    if (INTERIOR) {
-      A[k] = S::ld2(uin, (t.oy - hA + j) * W + (t.ox - hA + i));
-    } else {
-      const int gy = t.cy(t.oy - hA + j), gx = t.cx(t.ox - hA + i);
+    gy = INTERIOR ? t.oy - hA + j : t.cy(t.oy - hA + j);
+    gx = INTERIOR ? t.ox - hA + i : t.cx(t.ox - hA + i);
+  };
+  if (ADV) {
+    // a thread's slots in groups of G: the group's velocities in flight
+    // together, then its corners; cells and corners of the grid's outermost
+    // ring, whose values the walls make, are read once more through them
+    constexpr int N = (WA * HA + NT - 1) / NT, G = N < 4 ? N : 4;
+    auto ring = [&](int x, int y) { return x == 0 || y == 0 || x == W - 1 || y == t.H - 1; };
+#pragma unroll
+    for (int g0 = 0; g0 < N; g0 += G) {
+      int gx[G], gy[G];
+      float2 v[G];
+      uint8_t m[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        slot(min(tid + NT * (g0 + g), WA * HA - 1), gx[g], gy[g]);
+        v[g] = S::ld2(uin, gy[g] * W + gx[g]);
+        m[g] = mask[gy[g] * W + gx[g]];
+      }
+      Bilin c[G];
+      float2 lt[G], rt[G], lb[G], rb[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (ring(gx[g], gy[g])) v[g] = load_bc<S>(uin, gx[g], gy[g], W, t.H, adv.bc);
+        c[g] = bilinear_corners((float)gx[g] - (v[g].x * dt) * adv.speed,
+                                (float)gy[g] - (v[g].y * dt) * adv.speed, W, t.H);
+        lt[g] = S::ld2(uin, c[g].lt);
+        rt[g] = S::ld2(uin, c[g].rt);
+        lb[g] = S::ld2(uin, c[g].lb);
+        rb[g] = S::ld2(uin, c[g].rb);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (c[g].bx == 0 || c[g].by == 0 || c[g].tx == W - 1 || c[g].ty == t.H - 1) {
+          lt[g] = load_bc<S>(uin, c[g].bx, c[g].ty, W, t.H, adv.bc);
+          rt[g] = load_bc<S>(uin, c[g].tx, c[g].ty, W, t.H, adv.bc);
+          lb[g] = load_bc<S>(uin, c[g].bx, c[g].by, W, t.H, adv.bc);
+          rb[g] = load_bc<S>(uin, c[g].tx, c[g].by, W, t.H, adv.bc);
+        }
+        const float2 q = bilinear_mix<float2>(lt[g], rt[g], lb[g], rb[g], c[g].dx, c[g].dy);
+        const bool fluid = m[g] == 0;
+        typename S::s2 w;
+        S::st2(&w, 0, make_float2(fluid ? clampf(q.x * adv.diss, -1.0f, 1.0f) : 0.0f,
+                                  fluid ? clampf(q.y * adv.diss, -1.0f, 1.0f) : 0.0f));
+        if (tid + NT * (g0 + g) < WA * HA) A[tid + NT * (g0 + g)] = S::ld2(&w, 0);
+      }
+    }
+  } else {
+    for (int k = tid; k < WA * HA; k += NT) {
+      int gx, gy;
+      slot(k, gx, gy);
       A[k] = S::ld2(uin, gy * W + gx);
     }
   }
   __syncthreads();
 
   // 2. curl, shader.CalcVorticity.comp:21-26
-  for (int k = tid; k < WW * HW; k += 256) {
+  for (int k = tid; k < WW * HW; k += NT) {
     const int j = k / WW, i = k - j * WW;
     float2 vL, vR, vB, vT;
     if (INTERIOR) {
@@ -94,7 +154,7 @@ __device__ __forceinline__ void fused_tile_stages(
   __syncthreads();
 
   // 3. confinement, shader.ApplyVorticity.comp:26-39
-  for (int k = tid; k < WV * HV; k += 256) {
+  for (int k = tid; k < WV * HV; k += NT) {
     const int j = k / WV, i = k - j * WV;
     if (INTERIOR) {
       const int w = (j + 1) * WW + (i + 1);
@@ -116,7 +176,7 @@ __device__ __forceinline__ void fused_tile_stages(
   int hf = hV2;
   if (VISC) {
     constexpr int W3 = TX + 2, H3 = TY + 2;
-    for (int k = tid; k < W3 * H3; k += 256) {
+    for (int k = tid; k < W3 * H3; k += NT) {
       const int j = k / W3, i = k - j * W3;
       float2 L, R, B, T, c;
       if (INTERIOR) {
@@ -147,7 +207,7 @@ __device__ __forceinline__ void fused_tile_stages(
   // 5. divergence (Divergence.comp:22-40) and the first sweep from p = 0:
   //    ((((0+0)+0)+0) - b) * 0.25 = (0 - b) * 0.25 (Poisson.comp:37)
   const int Wf = TX + 2 * hf;
-  for (int k = tid; k < TX * TY; k += 256) {
+  for (int k = tid; k < TX * TY; k += NT) {
     const int j = k / TX, i = k - j * TX;
     const int gy = t.oy + j, gx = t.ox + i;
     if (!INTERIOR && (gy >= t.H || gx >= W)) continue;
@@ -189,14 +249,15 @@ __device__ __forceinline__ void fused_tile_stages(
   }
 }
 
-// One 64x16 output tile with origin (ox, oy); 256 threads as (64, 4).
+// One 64x16 output tile with origin (ox, oy); NT threads as (64, NT / 64).
 // Velocity, divergence and p1 are stored in format S; the chain is float32.
-template <class S = F32S>
+template <class S = F32S, bool ADV = false, int NT = 256>
 __device__ __forceinline__ void fused_vort_div_tile(
     int ox, int oy, const typename S::s2* __restrict__ uin,
     const uint8_t* __restrict__ mask, typename S::s2* __restrict__ uout,
     typename S::s1* __restrict__ div, typename S::s1* __restrict__ p1, int W,
-    int H, float dt, float scale, int viscous, float alpha, float rbeta) {
+    int H, float dt, float scale, int viscous, float alpha, float rbeta,
+    const Advect& adv = Advect{0, 0.0f, 0.0f, BcParams{0, 0, 0.0f}}) {
   __shared__ float2 A[(TX + 2 * HMAX) * (TY + 2 * HMAX)];
   __shared__ float Wc[(TX + 2 * HMAX - 2) * (TY + 2 * HMAX - 2)];
   __shared__ float2 V2[(TX + 2 * HMAX - 4) * (TY + 2 * HMAX - 4)];
@@ -205,21 +266,29 @@ __device__ __forceinline__ void fused_vort_div_tile(
   const bool interior = ox - h >= 0 && oy - h >= 0 && ox + TX + h <= W && oy + TY + h <= H;
   if (viscous) {
     if (interior)
-      fused_tile_stages<S, true, true>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
-                                       alpha, rbeta);
+      fused_tile_stages<S, true, true, ADV, NT>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
+                                            alpha, rbeta, adv);
     else
-      fused_tile_stages<S, true, false>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
-                                        alpha, rbeta);
+      fused_tile_stages<S, true, false, ADV, NT>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
+                                             alpha, rbeta, adv);
   } else {
     if (interior)
-      fused_tile_stages<S, false, true>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
-                                        alpha, rbeta);
+      fused_tile_stages<S, false, true, ADV, NT>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
+                                             alpha, rbeta, adv);
     else
-      fused_tile_stages<S, false, false>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
-                                         alpha, rbeta);
+      fused_tile_stages<S, false, false, ADV, NT>(A, Wc, V2, t, uin, mask, uout, div, p1, dt, scale,
+                                              alpha, rbeta, adv);
   }
 }
 
+// threads of a block of the kernels with the advection in front: with few tiles
+// the block's own latency counts and 1024 threads shorten it (128^2: 18 to 13 us
+// for the stages of a step, 1001 x 699, 704 tiles: 31 to 26); with many, blocks
+// of 256 overlap better (2048^2: 69 us a step of three simulators in turn
+// against 77)
+inline int advect_threads(int W, int H) {
+  return ((W + TX - 1) / TX) * ((H + TY - 1) / TY) <= 768 ? 1024 : 256;
+}
 
 }  // namespace fused
 }  // namespace nx

@@ -33,19 +33,19 @@ namespace {
 
 using jt::wave_sum;
 
-template <int ROWS, int WAVES, int COLS, bool RES>
+template <int ROWS, int WAVES, int COLS, bool RES, bool PROJ>
 __global__ void __launch_bounds__(WAVES * 64)
     __attribute__((amdgpu_waves_per_eu(jt::jacobi_waves_per_eu<ROWS * COLS>())))
     k_jacobi_tb(const float* __restrict__ pin, const float* __restrict__ b,
                 const uint8_t* __restrict__ mask, float* __restrict__ pout,
                 int W, int H, int k, int nx, int ny, double* __restrict__ red,
-                const int* __restrict__ done) {
+                const int* __restrict__ done, jt::Project<F32S> proj) {
   if (done != nullptr && *done != 0) return;  // block-uniform early exit
   // 1D grid of nx * ny tiles in XCD order; the partial-sum record is the
   // tile's row-major index
   const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, nx * ny);
-  jt::jacobi_tb_tile<ROWS, WAVES, COLS, F32S, false, RES>(t % nx, t / nx, nx, ny, pin, b, mask,
-                                                          pout, W, H, k, red, t);
+  jt::jacobi_tb_tile<ROWS, WAVES, COLS, F32S, false, RES, PROJ>(
+      t % nx, t / nx, nx, ny, pin, b, mask, pout, W, H, k, red, t, nullptr, proj);
 }
 
 // Exact FP64 residual of p (or of a zero guess when p == nullptr) plus the
@@ -177,14 +177,18 @@ __global__ void __launch_bounds__(256)
 template <int ROWS, int WAVES, int COLS>
 hipError_t launch_tb(const float* pin, const float* b, const uint8_t* mask,
                      float* pout, int W, int H, int k, double* red,
-                     const int* done, hipStream_t s) {
-  const int nx = jt::axis_tiles(W, 64 * COLS, k), ny = jt::axis_tiles(H, ROWS * WAVES, k);
-  if (red)
-    k_jacobi_tb<ROWS, WAVES, COLS, true><<<nx * ny, WAVES * 64, 0, s>>>(
-        pin, b, mask, pout, W, H, k, nx, ny, red, done);
+                     const int* done, const jt::Project<F32S>& proj, hipStream_t s) {
+  const int kt = proj.u ? k + 1 : k;
+  const int nx = jt::axis_tiles(W, 64 * COLS, kt), ny = jt::axis_tiles(H, ROWS * WAVES, kt);
+  if (proj.u)
+    k_jacobi_tb<ROWS, WAVES, COLS, false, true><<<nx * ny, WAVES * 64, 0, s>>>(
+        pin, b, mask, pout, W, H, k, nx, ny, red, done, proj);
+  else if (red)
+    k_jacobi_tb<ROWS, WAVES, COLS, true, false><<<nx * ny, WAVES * 64, 0, s>>>(
+        pin, b, mask, pout, W, H, k, nx, ny, red, done, proj);
   else
-    k_jacobi_tb<ROWS, WAVES, COLS, false><<<nx * ny, WAVES * 64, 0, s>>>(
-        pin, b, mask, pout, W, H, k, nx, ny, red, done);
+    k_jacobi_tb<ROWS, WAVES, COLS, false, false><<<nx * ny, WAVES * 64, 0, s>>>(
+        pin, b, mask, pout, W, H, k, nx, ny, red, done, proj);
   return hipGetLastError();
 }
 
@@ -232,18 +236,33 @@ int cheb_launch_blocks(int W, int H, JacobiCfg c) {
   return ((W + VX - 1) / VX) * ((H + VY - 1) / VY);
 }
 
+static hipError_t launch_shape(const float* pin, const float* b, const uint8_t* mask, float* pout,
+                               int W, int H, JacobiCfg c, double* red, const int* done,
+                               const jt::Project<F32S>& proj, hipStream_t s) {
+#define NX_TB_LAUNCH(R, WV, CL)                     \
+  if (c.rows == R && c.waves == WV && c.cols == CL) \
+    return launch_tb<R, WV, CL>(pin, b, mask, pout, W, H, c.k, red, done, proj, s);
+  NX_TB_SHAPES(NX_TB_LAUNCH)
+#undef NX_TB_LAUNCH
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_jacobi_tb(const float* pin, const float* b,
                             const uint8_t* mask, float* pout, int W, int H,
                             JacobiCfg c, double* red, const int* done,
                             hipStream_t s) {
   if (!jacobi_cfg_supported(c)) return hipErrorInvalidValue;
   if (c.seg > 0) return launch_jacobi_stream(pin, b, mask, pout, W, H, c, red, done, s);
-#define NX_TB_LAUNCH(R, WV, CL)                                              \
-  if (c.rows == R && c.waves == WV && c.cols == CL)                          \
-    return launch_tb<R, WV, CL>(pin, b, mask, pout, W, H, c.k, red, done, s);
-  NX_TB_SHAPES(NX_TB_LAUNCH)
-#undef NX_TB_LAUNCH
-  return hipErrorInvalidValue;
+  return launch_shape(pin, b, mask, pout, W, H, c, red, done,
+                      jt::Project<F32S>{nullptr, nullptr}, s);
+}
+
+hipError_t launch_jacobi_project(const float* pin, const float* b, const uint8_t* mask,
+                                 float* pout, float2* u, uint8_t* mask_next, int W, int H,
+                                 JacobiCfg c, hipStream_t s) {
+  if (!jacobi_cfg_supported(c) || c.seg > 0 || !u) return hipErrorInvalidValue;
+  return launch_shape(pin, b, mask, pout, W, H, c, nullptr, nullptr,
+                      jt::Project<F32S>{u, mask_next}, s);
 }
 
 hipError_t launch_center_rhs(float* b, float* p, const uint8_t* mask, int n,

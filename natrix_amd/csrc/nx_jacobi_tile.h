@@ -136,6 +136,14 @@ __device__ __forceinline__ void store_cols(typename S::s1* __restrict__ p, int i
   *reinterpret_cast<typename P::type*>(p + i) = t;
 }
 
+// The projection a tile runs on the pressure it ends with (SubtractGradient.
+// comp:24-46 and the obstacle clear): velocity in place, the next step's mask.
+template <class S>
+struct Project {
+  typename S::s2* u;
+  uint8_t* mask_next;
+};
+
 // ROWS x COLS cells per lane: lane `l` of wave `w` owns tile columns
 // [COLS*l, COLS*l + COLS) and tile rows [ROWS*w, ROWS*w + ROWS).
 // k sweeps on tile (bx, by) of the nx x ny tiles of a W x H grid; `rid` is
@@ -149,17 +157,23 @@ __device__ __forceinline__ void store_cols(typename S::s1* __restrict__ p, int i
 // residual r = b - A p of the stored iterate instead of a sweep, the other
 // k-1 passes are Jacobi sweeps of A e = r from e = 0, and the tile writes
 // the float32 pressure p + e to pout32 (pout is unused).
-template <int ROWS, int WAVES, int COLS, class S = F32S, bool CORR = false, bool RES = false>
+// PROJ: the tile also projects the velocity with the pressure it ends with
+// (p + e with CORR), which needs the pressure's neighbours: it owns what k + 1
+// sweeps would leave valid.
+template <int ROWS, int WAVES, int COLS, class S = F32S, bool CORR = false, bool RES = false,
+          bool PROJ = false>
 __device__ __forceinline__ void jacobi_tb_tile(
     int bx, int by, int nx, int ny, const typename S::s1* __restrict__ pin,
     const typename S::s1* __restrict__ b, const uint8_t* __restrict__ mask,
     typename S::s1* __restrict__ pout, int W, int H, int k,
-    double* __restrict__ red, int rid, float* __restrict__ pout32 = nullptr) {
+    double* __restrict__ red, int rid, float* __restrict__ pout32 = nullptr,
+    const Project<S>& proj = Project<S>{nullptr, nullptr}) {
   constexpr int EX = 64 * COLS, EY = ROWS * WAVES;
   const int lane = threadIdx.x & 63;
   // wave-uniform: a scalar register, so branches on it are scalar branches
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const AxisTile ax = axis_tile(bx, nx, W, EX, k), ay = axis_tile(by, ny, H, EY, k);
+  const int kt = PROJ ? k + 1 : k;
+  const AxisTile ax = axis_tile(bx, nx, W, EX, kt), ay = axis_tile(by, ny, H, EY, kt);
   const int tcol0 = COLS * lane;
   const int gx0 = ax.o + tcol0, gy0 = ay.o + wave * ROWS;
 
@@ -445,13 +459,45 @@ __device__ __forceinline__ void jacobi_tb_tile(
 #pragma unroll
         for (int c = 0; c < COLS; ++c) p[r][c] = np[r][c];
     }
+    if (PROJ) {
+      if (CORR) {
+        // the pressure the projection takes is the stored iterate + e
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+          for (int c = 0; c < COLS; ++c)
+            p[r][c] = S::ld(pin + (long long)min(gy0 + r, H - 1) * W, min(gx0 + c, W - 1)) +
+                      p[r][c];
+        publish(s & 1, p);
+      }
+      float prev[COLS], above[COLS];
+      collect(s & 1, prev, above);
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const int gy = gy0 + r;
+        if (gy < ay.own0 || gy >= ay.own1) continue;
+        const long long row = (long long)gy * W + ax.o;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+          float x1, x2, y1, y2;
+          neighbours(p, r, c, prev, above, x1, x2, y1, y2);
+          if (gx0 + c >= ax.own0 && gx0 + c < ax.own1) {
+            float2 v = S::ld2(proj.u + row, tcol0 + c);
+            v.x -= 0.5f * (x2 - x1);
+            v.y -= 0.5f * (y2 - y1);
+            S::st2(proj.u + row, tcol0 + c, v);
+            (proj.mask_next + row)[tcol0 + c] = (mask + row)[tcol0 + c] & MASK_PERSIST;
+          }
+        }
+      }
+    }
   };
 
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
   if (idle) {
-    for (int s = 0; s < k; ++s) __syncthreads();
+    for (int s = 0; s < kt; ++s) __syncthreads();
   } else if (special) {
     bool all = sol_lo == (1u << COLS) - 1 && sol_hi == (1u << COLS) - 1;
 #pragma unroll
@@ -480,7 +526,7 @@ __device__ __forceinline__ void jacobi_tb_tile(
 #pragma unroll
       for (int c = 0; c < COLS; ++c)
         if (gx0 + c >= ax.own0 && gx0 + c < ax.own1)
-          (pout32 + row)[tcol0 + c] = S::ld(pin + row, tcol0 + c) + p[r][c];
+          (pout32 + row)[tcol0 + c] = PROJ ? p[r][c] : S::ld(pin + row, tcol0 + c) + p[r][c];
     } else if (whole) {
       store_cols<S, COLS>(pout + row, tcol0, p[r]);
     } else {

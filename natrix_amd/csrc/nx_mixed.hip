@@ -33,30 +33,31 @@ __global__ void __launch_bounds__(256)
          advect_cell<S>(uin, mask, x, y, W, H, dt, speed, diss, bc));
 }
 
-template <class S>
-__global__ void __launch_bounds__(256)
+template <class S, bool ADV, int NT>
+__global__ void __launch_bounds__(NT)
     km_fused(const typename S::s2* __restrict__ uin,
              const uint8_t* __restrict__ mask, typename S::s2* __restrict__ uout,
              typename S::s1* __restrict__ div, typename S::s1* __restrict__ p1,
              int W, int H, float dt, float scale, int viscous, float alpha,
-             float rbeta) {
+             float rbeta, fused::Advect adv) {
   const int gx = (W + fused::TX - 1) / fused::TX;
   const int t = xcd_tile((int)blockIdx.x, gx * ((H + fused::TY - 1) / fused::TY));
-  fused::fused_vort_div_tile<S>((t % gx) * fused::TX, (t / gx) * fused::TY, uin, mask, uout,
-                                div, p1, W, H, dt, scale, viscous, alpha, rbeta);
+  fused::fused_vort_div_tile<S, ADV, NT>((t % gx) * fused::TX, (t / gx) * fused::TY, uin, mask,
+                                     uout, div, p1, W, H, dt, scale, viscous, alpha, rbeta, adv);
 }
 
-template <int ROWS, int WAVES, int COLS, class S, bool CORR>
+template <int ROWS, int WAVES, int COLS, class S, bool CORR, bool PROJ>
 __global__ void __launch_bounds__(WAVES * 64)
     __attribute__((amdgpu_waves_per_eu(jt::jacobi_waves_per_eu<ROWS * COLS>())))
     km_jacobi(const typename S::s1* __restrict__ pin,
               const typename S::s1* __restrict__ b,
               const uint8_t* __restrict__ mask, typename S::s1* __restrict__ pout,
-              float* __restrict__ pout32, int W, int H, int k, int nx, int ny) {
+              float* __restrict__ pout32, int W, int H, int k, int nx, int ny,
+              jt::Project<S> proj) {
   // 1D grid of nx * ny tiles in XCD order
   const int t = xcd_tile<XCD_RUNS>((int)blockIdx.x, nx * ny);
-  jt::jacobi_tb_tile<ROWS, WAVES, COLS, S, CORR>(t % nx, t / nx, nx, ny, pin, b, mask, pout, W,
-                                                 H, k, nullptr, 0, pout32);
+  jt::jacobi_tb_tile<ROWS, WAVES, COLS, S, CORR, false, PROJ>(
+      t % nx, t / nx, nx, ny, pin, b, mask, pout, W, H, k, nullptr, 0, pout32, proj);
 }
 
 template <class S>
@@ -124,27 +125,33 @@ hipError_t mixed_dispatch_advect(const void* uin, void* uout, const uint8_t* mas
 template <int R, int WV, int CL, class S>
 hipError_t mixed_tb(const void* pin, const void* b, const uint8_t* mask,
                     void* pout, float* pout32, int W, int H, int k, bool corr,
-                    hipStream_t s) {
-  const int nx = jt::axis_tiles(W, 64 * CL, k), ny = jt::axis_tiles(H, R * WV, k);
+                    const jt::Project<S>& proj, hipStream_t s) {
+  const int kt = proj.u ? k + 1 : k;
+  const int nx = jt::axis_tiles(W, 64 * CL, kt), ny = jt::axis_tiles(H, R * WV, kt);
   const dim3 grid(nx * ny);
-  if (corr)
-    km_jacobi<R, WV, CL, S, true><<<grid, WV * 64, 0, s>>>(
-        (const typename S::s1*)pin, (const typename S::s1*)b, mask,
-        (typename S::s1*)pout, pout32, W, H, k, nx, ny);
+  const auto* p = (const typename S::s1*)pin;
+  const auto* bs = (const typename S::s1*)b;
+  auto* po = (typename S::s1*)pout;
+  if (corr && proj.u)
+    km_jacobi<R, WV, CL, S, true, true>
+        <<<grid, WV * 64, 0, s>>>(p, bs, mask, po, pout32, W, H, k, nx, ny, proj);
+  else if (corr)
+    km_jacobi<R, WV, CL, S, true, false>
+        <<<grid, WV * 64, 0, s>>>(p, bs, mask, po, pout32, W, H, k, nx, ny, proj);
   else
-    km_jacobi<R, WV, CL, S, false><<<grid, WV * 64, 0, s>>>(
-        (const typename S::s1*)pin, (const typename S::s1*)b, mask,
-        (typename S::s1*)pout, pout32, W, H, k, nx, ny);
+    km_jacobi<R, WV, CL, S, false, false>
+        <<<grid, WV * 64, 0, s>>>(p, bs, mask, po, pout32, W, H, k, nx, ny, proj);
   return hipGetLastError();
 }
 
 template <class S>
 hipError_t mixed_tb_shape(const void* pin, const void* b, const uint8_t* mask,
                           void* pout, float* pout32, int W, int H, JacobiCfg c,
-                          bool corr, hipStream_t s) {
+                          bool corr, void* u, uint8_t* mask_next, hipStream_t s) {
+  const jt::Project<S> proj{(typename S::s2*)u, mask_next};
 #define NX_MTB(R, WV, CL)                                                 \
   if (c.rows == R && c.waves == WV && c.cols == CL)                       \
-    return mixed_tb<R, WV, CL, S>(pin, b, mask, pout, pout32, W, H, c.k, corr, s);
+    return mixed_tb<R, WV, CL, S>(pin, b, mask, pout, pout32, W, H, c.k, corr, proj, s);
   NX_MTB(4, 8, 1)
   NX_MTB(4, 16, 1)
   NX_MTB(8, 8, 1)
@@ -181,23 +188,46 @@ hipError_t launch_m_advect(int st, const void* uin, void* uout, const uint8_t* m
 template <class S>
 static hipError_t fused_m(const void* uin, const uint8_t* mask, void* uout, void* div,
                           void* p1, int W, int H, float dt, float scale,
-                          int viscous, float alpha, float rbeta, hipStream_t s) {
+                          int viscous, float alpha, float rbeta, const fused::Advect& adv,
+                          hipStream_t s) {
   const dim3 grid(((W + fused::TX - 1) / fused::TX) * ((H + fused::TY - 1) / fused::TY), 1, 1);
-  km_fused<S><<<grid, dim3(64, 4), 0, s>>>(
-      (const typename S::s2*)uin, mask, (typename S::s2*)uout,
-      (typename S::s1*)div, (typename S::s1*)p1, W, H, dt, scale, viscous, alpha,
-      rbeta);
+  const auto* u = (const typename S::s2*)uin;
+  auto* uo = (typename S::s2*)uout;
+  auto* d = (typename S::s1*)div;
+  auto* p = (typename S::s1*)p1;
+  if (!adv.on)
+    km_fused<S, false, 256><<<grid, dim3(64, 4), 0, s>>>(u, mask, uo, d, p, W, H, dt, scale,
+                                                         viscous, alpha, rbeta, adv);
+  else if (fused::advect_threads(W, H) == 1024)
+    km_fused<S, true, 1024><<<grid, dim3(64, 16), 0, s>>>(u, mask, uo, d, p, W, H, dt, scale,
+                                                          viscous, alpha, rbeta, adv);
+  else
+    km_fused<S, true, 256><<<grid, dim3(64, 4), 0, s>>>(u, mask, uo, d, p, W, H, dt, scale,
+                                                        viscous, alpha, rbeta, adv);
   return hipGetLastError();
 }
 
 hipError_t launch_m_fused(int st, const void* uin, const uint8_t* mask, void* uout,
                           void* div, void* p1, int W, int H, float dt, float scale,
                           int viscous, float alpha, float rbeta, hipStream_t s) {
+  const fused::Advect off{};
   return NX_BY_STORAGE(st,
                        fused_m<BF16S>(uin, mask, uout, div, p1, W, H, dt, scale,
-                                      viscous, alpha, rbeta, s),
+                                      viscous, alpha, rbeta, off, s),
                        fused_m<F16S>(uin, mask, uout, div, p1, W, H, dt, scale,
-                                     viscous, alpha, rbeta, s));
+                                     viscous, alpha, rbeta, off, s));
+}
+
+hipError_t launch_m_advect_fused(int st, const void* uin, const uint8_t* mask, void* uout,
+                                 void* div, void* p1, int W, int H, float dt, float speed,
+                                 float diss, BcParams bc, float scale, int viscous, float alpha,
+                                 float rbeta, hipStream_t s) {
+  const fused::Advect adv{1, speed, diss, bc};
+  return NX_BY_STORAGE(st,
+                       fused_m<BF16S>(uin, mask, uout, div, p1, W, H, dt, scale,
+                                      viscous, alpha, rbeta, adv, s),
+                       fused_m<F16S>(uin, mask, uout, div, p1, W, H, dt, scale,
+                                     viscous, alpha, rbeta, adv, s));
 }
 
 hipError_t launch_m_jacobi(int st, const void* pin, const void* b, const uint8_t* mask,
@@ -205,8 +235,17 @@ hipError_t launch_m_jacobi(int st, const void* pin, const void* b, const uint8_t
                            bool corr, hipStream_t s) {
   if (!jacobi_cfg_supported(c)) return hipErrorInvalidValue;
   return NX_BY_STORAGE(
-      st, mixed_tb_shape<BF16S>(pin, b, mask, pout, pout32, W, H, c, corr, s),
-      mixed_tb_shape<F16S>(pin, b, mask, pout, pout32, W, H, c, corr, s));
+      st, mixed_tb_shape<BF16S>(pin, b, mask, pout, pout32, W, H, c, corr, nullptr, nullptr, s),
+      mixed_tb_shape<F16S>(pin, b, mask, pout, pout32, W, H, c, corr, nullptr, nullptr, s));
+}
+
+hipError_t launch_m_correct_project(int st, const void* pin, const void* b, const uint8_t* mask,
+                                    float* pout32, void* u, uint8_t* mask_next, int W, int H,
+                                    JacobiCfg c, hipStream_t s) {
+  if (!jacobi_cfg_supported(c) || !u) return hipErrorInvalidValue;
+  return NX_BY_STORAGE(
+      st, mixed_tb_shape<BF16S>(pin, b, mask, nullptr, pout32, W, H, c, true, u, mask_next, s),
+      mixed_tb_shape<F16S>(pin, b, mask, nullptr, pout32, W, H, c, true, u, mask_next, s));
 }
 
 template <class S>

@@ -140,5 +140,5 @@ struct TimeScope {
 namespace nx {
 // `sweeps` Jacobi sweeps of the simulator's pressure with launch shape c
 // (tile or streaming kernels, k sweeps per launch), on its stream
-int run_jacobi_tb(::nx_sim* s, int sweeps, JacobiCfg c);
+int run_jacobi_tb(::nx_sim* s, int sweeps, JacobiCfg c, float2* u = nullptr);
 }  // namespace nx

@@ -1,0 +1,62 @@
+"""The step's merged form (advection inside the following stages' kernel, the
+projection inside the last Jacobi launch) against the oracle and, bitwise,
+against the separate launches that a timed simulator runs."""
+import numpy as np
+import pytest
+
+from natrix_amd import FluidSimulator
+from oracle import fluid as F
+
+pytestmark = pytest.mark.gpu
+
+BC = {"reference": F.BC_REFERENCE, "free_slip": F.BC_FREE_SLIP, "inflow": F.BC_INFLOW}
+
+
+def _pair(w, h, storage, bc, visc, iters, seed):
+    rng = np.random.default_rng(seed)
+    # large velocities: back-traces reach the walls and leave the grid
+    u = (1.5 * rng.standard_normal((h, w, 2))).astype(np.float32)
+    solid = rng.random((h, w)) < 0.08
+    out = []
+    for timed in (False, True):
+        sim = FluidSimulator(w, h, storage=storage, bc_mode=bc)
+        sim.vorticity, sim.viscosity, sim.iterations = 0.3, visc, iters
+        sim.set_obstacle_map(solid)
+        sim.upload("velocity", u)
+        if timed:
+            sim.set_timing(True)
+        out.append(sim)
+    return out, u, solid
+
+
+# tiles of the stages are 64 x 16 (halo 3 or 4): below, at and above one and two
+# tiles, narrower than the halo, and enough tiles for the 256-thread form
+@pytest.mark.parametrize("w,h", [(3, 3), (64, 16), (65, 17), (63, 40), (130, 33), (200, 7),
+                                 (1300, 700)])
+@pytest.mark.parametrize("bc,visc", [("reference", 0.0), ("free_slip", 0.1), ("inflow", 0.0)])
+@pytest.mark.parametrize("storage", ["f32", "bf16", "f16"])
+def test_merged_equals_separate(gpu, w, h, bc, visc, storage):
+    sims, u, solid = _pair(w, h, storage, bc, visc, 14, w + h)
+    for step in range(2):
+        for sim in sims:
+            sim.add_circle_obstacle((0.3, 0.6), 0.2 * min(w, h))
+            sim.update(1 / 60)
+        for f in ("velocity", "pressure", "divergence", "mask"):
+            a, b = (sim.download(f) for sim in sims)
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (step, f)
+    for sim in sims:
+        sim.destroy()
+
+
+@pytest.mark.parametrize("iters", [1, 2, 25, 26])
+def test_merged_step_is_the_oracle(gpu, iters):
+    """One sweep (no launch to carry the projection) and whole or uneven launches."""
+    w, h = 150, 90
+    (sim, _), u, solid = _pair(w, h, "f32", "inflow", 0.0, iters, 7)
+    sim.update(1 / 60)
+    prm = F.Params(vorticity=0.3, viscosity=0.0, iterations=iters, bc_mode=F.BC_INFLOW)
+    ref, p, _, _ = F.step(u, np.zeros((h, w), np.float32), np.zeros((h, w, 2), np.float32),
+                          np.float32(1 / 60), prm, persistent=solid)
+    assert np.array_equal(sim.download("velocity"), ref)
+    assert np.array_equal(sim.download("pressure"), p)
+    sim.destroy()
