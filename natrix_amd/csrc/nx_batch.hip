@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256)
                   const uint8_t* __restrict__ mask, float dt) {
   NX_BATCH_CELL_LOOP(prefix, S, total)
     qout[pos] = advect_dye_cell(qin + d.off, u + d.off, mask + d.off, x, y,
-                                d.W, d.H, d.W, d.H, dt, d.dye_speed, d.dye_diss);
+                                d.W, d.H, d.W, d.H, 1.0f, 1.0f, dt, d.dye_speed, d.dye_diss);
   }
 }
 

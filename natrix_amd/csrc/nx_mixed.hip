@@ -79,12 +79,12 @@ __global__ void __launch_bounds__(256)
                   typename S::s1* __restrict__ qout,
                   const typename S::s2* __restrict__ u,
                   const uint8_t* __restrict__ mask, int Wp, int Hp, int Wv,
-                  int Hv, float dt, float speed, float diss) {
+                  int Hv, float sx, float sy, float dt, float speed, float diss) {
   int x, y;
   cell_of(x, y, Wp, Hp);
   if (x >= Wp || y >= Hp) return;
   S::st(qout, y * Wp + x,
-        advect_dye_cell<S>(qin, u, mask, x, y, Wp, Hp, Wv, Hv, dt, speed, diss));
+        advect_dye_cell<S>(qin, u, mask, x, y, Wp, Hp, Wv, Hv, sx, sy, dt, speed, diss));
 }
 
 struct SplatBatchM {
@@ -270,7 +270,7 @@ static hipError_t dye_m(const void* qin, void* qout, const void* u,
                         float dt, float speed, float diss, hipStream_t s) {
   km_advect_dye<S><<<grid2d(Wp, Hp), dim3(BX, BY), 0, s>>>(
       (const typename S::s1*)qin, (typename S::s1*)qout, (const typename S::s2*)u,
-      mask, Wp, Hp, Wv, Hv, dt, speed, diss);
+      mask, Wp, Hp, Wv, Hv, (float)Wp / (float)Wv, (float)Hp / (float)Hv, dt, speed, diss);
   return hipGetLastError();
 }
 

@@ -228,11 +228,11 @@ __global__ void __launch_bounds__(256)
     k_advect_dye(const float* __restrict__ qin, float* __restrict__ qout,
                  const float2* __restrict__ u,
                  const uint8_t* __restrict__ mask, int Wp, int Hp, int Wv,
-                 int Hv, float dt, float speed, float diss) {
+                 int Hv, float sx, float sy, float dt, float speed, float diss) {
   int x, y;
   if (!cell(x, y, Wp, Hp)) return;
   qout[y * Wp + x] =
-      advect_dye_cell(qin, u, mask, x, y, Wp, Hp, Wv, Hv, dt, speed, diss);
+      advect_dye_cell(qin, u, mask, x, y, Wp, Hp, Wv, Hv, sx, sy, dt, speed, diss);
 }
 
 // ---------------------------------------------------------------- F4
@@ -363,7 +363,8 @@ hipError_t launch_advect_dye(const float* qin, float* qout, const float2* u,
                              int Hv, float dt, float speed, float diss,
                              hipStream_t s) {
   NX_LAUNCH(k_advect_dye<<<grid2d(Wp, Hp), dim3(BX, BY), 0, s>>>(
-      qin, qout, u, mask, Wp, Hp, Wv, Hv, dt, speed, diss));
+      qin, qout, u, mask, Wp, Hp, Wv, Hv, (float)Wp / (float)Wv, (float)Hp / (float)Hv, dt, speed,
+      diss));
 }
 hipError_t launch_add_dye(const float* qin, float* qout, int W, int H,
                           float px, float py, float val, float r,

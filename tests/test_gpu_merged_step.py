@@ -60,3 +60,19 @@ def test_merged_step_is_the_oracle(gpu, iters):
     assert np.array_equal(sim.download("velocity"), ref)
     assert np.array_equal(sim.download("pressure"), p)
     sim.destroy()
+
+
+def test_splats_far_and_near_a_zero_weight(gpu):
+    """Weights around the last one that does not round to zero (10.2 radii)."""
+    w, h = 400, 24
+    rng = np.random.default_rng(5)
+    u = rng.standard_normal((h, w, 2)).astype(np.float32)
+    u[::3] = -0.0
+    sim = FluidSimulator(w, h)
+    splats = [(0.02, 0.5, 1e30, -1e30, 7.0, 0.0), (0.9, 0.3, -2.0, 1e38, 11.5, 0.0),
+              (-4.0, 0.5, 1.0, 1.0, 3.0, 0.0)]
+    sim.upload("velocity", u)
+    sim.add_splats(splats)
+    ref, _ = F.gaussian_splat(u, None, [tuple(np.float32(v) for v in s) for s in splats])
+    assert np.array_equal(sim.download("velocity").view(np.uint32), ref.view(np.uint32))
+    sim.destroy()
