@@ -260,7 +260,8 @@ int nx_refine_end(nx_sim* sim);
 int nx_step_finish(nx_sim* sim);
 
 /* Capture the fixed-iteration step into a HIP graph and replay it on later
- * nx_update calls with the same dt and parameters (on = 1). */
+ * nx_update calls with the same dt and parameters (on = 1); steps of a few
+ * launches, which cost less enqueued than replayed, are enqueued. */
 int nx_set_graph(nx_sim* sim, int on);
 
 /* ---- per-stage entry points (one reference shader each), operating on the

@@ -306,6 +306,15 @@ static bool step_merged(const nx_sim* s, bool tolerance) {
          (s->storage != ST_F32 || (s->prm.iterations > 1 && s->prm.jacobi_seg == 0));
 }
 
+// launches of a fixed-iteration fused step
+static int step_launches(const nx_sim* s) {
+  const nx_params& P = s->prm;
+  const int sweeps = P.iterations - 1;
+  const int jacobi = sweeps > 0 ? (sweeps + P.jacobi_k - 1) / P.jacobi_k : 0;
+  return (step_merged(s, false) ? 1 : 3) + jacobi + (s->storage != ST_F32 ? 1 : 0) +
+         (s->dye[0] && P.dye_in_step ? 1 : 0);
+}
+
 static void viscosity_of(const nx_params& P, int& viscous, float& alpha, float& rbeta) {
   viscous = P.viscosity > 0.0f;
   alpha = rbeta = 0.0f;
@@ -838,7 +847,8 @@ int nx_update(nx_sim* s, float dt) {
   const nx_params& P = s->prm;
   if (!P.fused) return step_reference_order(s, dt);
   if (P.tol > 0) return step_fused_enqueue(s, dt, true);
-  if (!s->graph_on || s->timing) return step_fused_enqueue(s, dt, false);
+  if (!s->graph_on || s->timing || step_launches(s) < GRAPH_MIN_LAUNCHES)
+    return step_fused_enqueue(s, dt, false);
   // graph replay keyed by the buffer parities and by dt + parameters
   const bool dye_step = s->dye[0] && P.dye_in_step;
   const int par = s->vcur | (s->mcur << 1) | (dye_step ? (s->dcur << 2) : 0);

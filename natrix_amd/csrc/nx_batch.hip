@@ -388,6 +388,13 @@ static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c, bool project = fal
 // or there is no further sweep
 static bool batch_step_merged(const nx_batch* b) { return !b->timing && b->prm.iterations > 1; }
 
+static int batch_step_launches(const nx_batch* b) {
+  const int sweeps = b->prm.iterations - 1;
+  const int jacobi = sweeps > 0 ? (sweeps + b->prm.jacobi_k - 1) / b->prm.jacobi_k : 0;
+  return (batch_step_merged(b) ? 1 : 3) + jacobi + (b->splats.empty() ? 0 : 1) +
+         (b->dye[0] ? 1 : 0);
+}
+
 // every prefix table a step needs (no allocation inside a capture)
 static int batch_step_tables(nx_batch* b) {
   const nx_params& P = b->prm;
@@ -632,7 +639,8 @@ int nx_batch_update(nx_batch* b, float dt) {
   if (!b) return bfail(NX_ERR_ARG, "null batch");
   NXB_TRY(sync_scenes(b));
   const nx_params& P = b->prm;
-  if (!b->graph_on || b->timing) return batch_step(b, dt);
+  if (!b->graph_on || b->timing || batch_step_launches(b) < GRAPH_MIN_LAUNCHES)
+    return batch_step(b, dt);
   const bool dye = b->dye[0] != nullptr;
   const int par = b->vcur | (b->mcur << 1) | (dye ? (b->dcur << 2) : 0);
   if (!b->graph[par] || b->graph_dt[par] != dt ||

@@ -80,6 +80,12 @@ struct JacobiCfg {
   int cols;     // columns per lane
   int seg = 0;  // > 0: streaming kernel, output rows per workgroup segment
 };
+// A captured step is replayed only from this many launches on: a launch costs the
+// host 2.7 us, a replay 15 us and 1 us a node (256^2, 40 sweeps, 4 launches: 13.7
+// us a step enqueued, 21.9 replayed, three simulators in turn; 1024^2, 5
+// launches: 66.7 and 68.5), and the results are the same.
+constexpr int GRAPH_MIN_LAUNCHES = 10;
+
 // sweeps per launch that spread `sweeps` evenly over ceil(sweeps / k) launches
 inline int jacobi_even_k(int sweeps, int k) {
   if (sweeps <= 0) return k;

@@ -62,6 +62,28 @@ def test_merged_step_is_the_oracle(gpu, iters):
     sim.destroy()
 
 
+@pytest.mark.parametrize("storage", ["f32", "f16"])
+def test_graph_of_many_launches_replays(gpu, storage):
+    """Steps of ten launches and more are captured; replays, with other work and
+    waits between them, give the eager steps."""
+    w, h = 140, 70
+    sims, u, _ = _pair(w, h, storage, "free_slip", 0.0, 40, 11)
+    sims[1].set_timing(False)
+    for sim in sims:
+        sim.jacobi_tile = (3, 4, 8, 2)
+    sims[0].use_graph = True
+    for step in range(7):
+        for sim in sims:
+            if step % 3 == 2:
+                sim.add_splats([(0.4, 0.5, 0.7, -0.3, 4.0, 0.0)])
+            sim.update(1 / 60)
+        for f in ("velocity", "pressure", "mask"):
+            a, b = (sim.download(f) for sim in sims)
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (step, f)
+    for sim in sims:
+        sim.destroy()
+
+
 def test_splats_far_and_near_a_zero_weight(gpu):
     """Weights around the last one that does not round to zero (10.2 radii)."""
     w, h = 400, 24
