@@ -114,3 +114,31 @@ def test_head_backward(gpu, pixels, c):
     assert bool(((wg.grad.double().cpu() - terms.sum(0)).abs() <= bound).all())
     assert abs(float(bg.grad) - float(dout.double().sum())) <= \
         pixels * 2.0 ** -24 * float(dout.double().abs().sum())
+
+
+@pytest.mark.parametrize("n,h,w,ca,cb", [(1, 2, 2, 8, 16), (2, 6, 10, 64, 32), (1, 4, 2, 5, 3),
+                                         (3, 8, 4, 24, 12)])
+def test_movers_wide_and_single(gpu, n, h, w, ca, cb):
+    """Pool, upsample and concat, forward and backward, with channel counts that
+    take 16-byte accesses and counts that do not, against torch on the CPU."""
+    g = torch.Generator().manual_seed(n * h * w + ca)
+    x = torch.randn(n, h, w, ca, generator=g).to(BF)
+    s = torch.randn(n, h, w, cb, generator=g).to(BF)
+    d = torch.randn(n, h, w, ca, generator=g).to(BF)
+    xg, sg = (t.cuda().requires_grad_(True) for t in (x, s))
+    p = U.Pool2Fn.apply(xg)
+    f = x.float().view(n, h // 2, 2, w // 2, 2, ca)
+    want = (((f[:, :, 0, :, 0] + f[:, :, 0, :, 1]) + f[:, :, 1, :, 0]) + f[:, :, 1, :, 1]) * 0.25
+    assert torch.equal(p.detach().cpu(), want.to(BF))
+    u = U.Up2Fn.apply(p)
+    assert torch.equal(u.detach().cpu(),
+                       want.to(BF).repeat_interleave(2, 1).repeat_interleave(2, 2))
+    y = U.ConcatFn.apply(u, sg)
+    assert torch.equal(y.detach().cpu(), torch.cat([u.detach().cpu(), s], 3))
+    dy = torch.cat([d, s], 3).contiguous()
+    y.backward(dy.cuda())
+    assert torch.equal(sg.grad.cpu(), s)
+    e = d.float().view(n, h // 2, 2, w // 2, 2, ca)
+    up = (((e[:, :, 0, :, 0] + e[:, :, 0, :, 1]) + e[:, :, 1, :, 0]) + e[:, :, 1, :, 1]).to(BF)
+    pool = (up.float() * 0.25).to(BF)
+    assert torch.equal(xg.grad.cpu(), pool.repeat_interleave(2, 1).repeat_interleave(2, 2))
