@@ -12,7 +12,7 @@
 #include <math.h>
 
 #include "../../include/natrix.h"
-#include "nx_jacobi_tile.h"
+#include "nx_cheb_tile.h"
 #include "nx_kernels.h"
 #include "nx_sim.h"
 
@@ -437,191 +437,26 @@ __global__ void __launch_bounds__(256)
   pout[pos] = p + w * (jac - p);
 }
 
-// The Chebyshev smoothing of k_coarse_smooth<true> spread over 2D tiles:
-// a workgroup of CT_WAVES waves holds a 64 x CT_EY tile (lane l column l,
-// wave w rows CT_ROWS w .. CT_ROWS w + CT_ROWS - 1), and a launch runs up
-// to CB_T iterations on it (plus, at the first launch, the initial
-// residual).  A tile overlaps its neighbours by CT_HALO = CB_T + 1 cells on
-// every side, whose values go stale one cell per stencil, and stores its
-// CT_VX x CT_VY interior: at 128 x 128, 4 x 22 workgroups of 1024 threads,
-// 2 cells per lane (the shape and CB_T timed fastest on the 2048^2 learned
-// step among 8 to 16 iterations per launch and 4 to 16 waves).  Launch
-// boundaries are the only global synchronisation.  Every cell sees the
-// operations of the single-workgroup kernel in the same order, so x is
-// bitwise the same; wavefronts whose cells have no solid or out-of-grid
-// neighbour (the inner tiles away from obstacles) take a select-free
-// stencil with the same sums.  Theta and the
-// coefficients of the launch's iterations (cf) come from the host, computed
-// by the same float32 operations (IEEE single on both sides).
-constexpr int CB_T = 12, CT_ROWS = 2, CT_WAVES = 16, CT_HALO = CB_T + 1;
-constexpr int CT_EY = CT_ROWS * CT_WAVES, CT_VX = 64 - 2 * CT_HALO, CT_VY = CT_EY - 2 * CT_HALO;
-static_assert(CT_VX > 0 && CT_VY > 0, "coarse tile smaller than its halo");
+// The Chebyshev smoothing of k_coarse_smooth<true> on tiles of many workgroups
+// (nx_cheb_tile.h): the same operations in the same order, so x is bitwise the
+// same.  Launch boundaries are the only global synchronisation.  A pass is bound
+// by the exchange (LDS round trip and barrier, 0.3 us), then by the slowest
+// wave's cells, so a lane holds three cells and one launch runs many
+// iterations: 100 of them at 128 x 128, face weights open / cut by a circle, in
+// us: 70 / 71 with 64 x 32 tiles at 12 a launch and a halo beyond the grid's
+// edges (the form before), 67 / 79 with these tiles at 2 rows, 57 / 71 at 3 rows
+// and 20 a launch, 56 / 70 at 4 rows and 25 (with a padded edge 71, 69, 61, 67);
+// two columns a lane 85 / 133.
+constexpr int CT_ROWS = 3, CT_WAVES = 16, CT_COLS = 1;
+// iterations a launch: the halos of 20 leave 6 rows of a tile's 48, which pays
+// while all tiles run at once (two workgroups a CU), else 12
+constexpr int CT_T = 20, CT_T_MANY = 12, CT_TILES = 512;
+constexpr int CB_T = 12;  // plain operator: up to here one resident workgroup does it
 
-// FACES: the face-weighted operator of k_coarse_faces.  A neighbour across
-// a face of weight w enters the sum as the centre c when w = 0 (as a solid
-// neighbour does), as itself when w = 1, and as fma(w, v - c, c) between,
-// so that the sum minus 4 c is the sum of w (v - c); a cell whose faces
-// are all shut or all open sees the operations of the plain kernel.
 template <bool FACES>
 __global__ void __launch_bounds__(64 * CT_WAVES)
-    k_coarse_cheb_tile(const float* __restrict__ xin, const float* __restrict__ rin,
-                       const float* __restrict__ din, float* __restrict__ xout,
-                       float* __restrict__ rout, float* __restrict__ dout,
-                       const float* __restrict__ rhs, const uint8_t* __restrict__ mc,
-                       const float* __restrict__ faces, int Wc, int Hc, int s0, int T,
-                       float theta, ChebCoef cf) {
-  constexpr int R = CT_ROWS;
-  const int lane = threadIdx.x & 63;
-  // wave-uniform: a scalar register, so branches on it are scalar branches
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int gx = (int)blockIdx.x * CT_VX - CT_HALO + lane;
-  const int gy0 = (int)blockIdx.y * CT_VY - CT_HALO + wave * R;
-  const bool first = s0 == 0;
-  // Every load is unconditional, from a clamped in-grid address, issued
-  // before the first use: x, r (b at the first launch) and d of the lane's
-  // cells, and the mask of its column over the rows gy0 - 1 .. gy0 + R; the
-  // neighbours' flags to the left and right come from the adjacent lanes,
-  // and a cell outside the grid counts as solid.
-  const float* rsrc = first ? rhs : rin;
-  const int cx = min(max(gx, 0), Wc - 1);
-  float lx[R], lr[R], ld[R];
-  uint8_t lm[R + 2];
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int pos = min(max(gy0 + i, 0), Hc - 1) * Wc + cx;
-    lx[i] = xin[pos];
-    lr[i] = rsrc[pos];
-    ld[i] = din[pos];
-  }
-#pragma unroll
-  for (int i = 0; i < R + 2; ++i) lm[i] = mc[min(max(gy0 - 1 + i, 0), Hc - 1) * Wc + cx];
-  const bool col_in = gx >= 0 && gx < Wc;
-  int sf[R + 2];  // solid flags of rows gy0 - 1 + i
-#pragma unroll
-  for (int i = 0; i < R + 2; ++i) {
-    const int gy = gy0 - 1 + i;
-    sf[i] = (col_in && gy >= 0 && gy < Hc) ? lm[i] != 0 : 1;
-  }
-  float x[R], r[R], d[R], lv[R];
-  int code[R];  // bit 0: left, 1: right, 2: up (y-1), 3: down (y+1) solid
-  // FACES: the weights of the cell's four faces and which are partial
-  float wl[FACES ? R : 1], wr[FACES ? R : 1], wu[FACES ? R : 1], wd[FACES ? R : 1];
-  int part[FACES ? R : 1];
-  float fe[FACES ? R : 1], fs[FACES ? R + 1 : 1];
-  if (FACES) {
-    const int n = Wc * Hc;
-#pragma unroll
-    for (int i = 0; i < R; ++i) fe[i] = faces[min(max(gy0 + i, 0), Hc - 1) * Wc + cx];
-#pragma unroll
-    for (int i = 0; i < R + 1; ++i) fs[i] = faces[n + min(max(gy0 - 1 + i, 0), Hc - 1) * Wc + cx];
-  }
-  bool any = false;
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int gy = gy0 + i;
-    const bool in = col_in && gy >= 0 && gy < Hc;
-    x[i] = in ? lx[i] : 0.0f;
-    r[i] = in ? lr[i] : 0.0f;
-    d[i] = (in && !first) ? ld[i] : 0.0f;
-    if (FACES) {
-      // a cell outside the grid, and a face on the grid's edge, is shut;
-      // the west face is the left lane's east face (lane 0 keeps its own:
-      // a halo cell)
-      wr[i] = (in && gx < Wc - 1) ? fe[i] : 0.0f;
-      wd[i] = (in && gy < Hc - 1) ? fs[i + 1] : 0.0f;
-      wu[i] = (in && gy > 0) ? fs[i] : 0.0f;
-      wl[i] = jt::lane_from_left(wr[i]);
-      if (!in) wl[i] = 0.0f;
-      code[i] = (wl[i] == 0.0f ? 1 : 0) | (wr[i] == 0.0f ? 2 : 0) | (wu[i] == 0.0f ? 4 : 0) |
-                (wd[i] == 0.0f ? 8 : 0);
-      part[i] = (wl[i] > 0.0f && wl[i] < 1.0f ? 1 : 0) | (wr[i] > 0.0f && wr[i] < 1.0f ? 2 : 0) |
-                (wu[i] > 0.0f && wu[i] < 1.0f ? 4 : 0) | (wd[i] > 0.0f && wd[i] < 1.0f ? 8 : 0);
-      any |= (code[i] | part[i]) != 0;
-    } else {
-      // the lane shifts run with every lane active; lanes 0 and 63 keep
-      // their own flag, which only affects halo cells
-      const int lnb = jt::ilane_from_left(sf[i + 1]);
-      const int rnb = jt::ilane_from_right(sf[i + 1]);
-      code[i] = lnb | (rnb << 1) | (sf[i] << 2) | (sf[i + 2] << 3);
-      any |= code[i] != 0;
-    }
-  }
-  const bool special = __any(any);  // wave-uniform
-
-  __shared__ float top[2][CT_WAVES][64], bot[2][CT_WAVES][64];
-  int buf = 0;
-  // out = L v: ((u + l) + r) + d - 4 c, a solid or out-of-grid neighbour
-  // replaced by the centre; every thread of the block calls it
-  auto lap = [&](const float (&v)[R], float (&out)[R]) {
-    top[buf][wave][lane] = v[0];
-    bot[buf][wave][lane] = v[R - 1];
-    __syncthreads();
-    // the rows beyond the tile's first and last are halo: any finite value
-    const float up0 = bot[buf][wave > 0 ? wave - 1 : wave][lane];
-    const float dn0 = top[buf][wave < CT_WAVES - 1 ? wave + 1 : wave][lane];
-    buf ^= 1;
-    if (special) {
-#pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float c = v[i];
-        const float fl = jt::lane_from_left(c), fr = jt::lane_from_right(c);
-        const float U = i > 0 ? v[i - 1] : up0;
-        const float D = i < R - 1 ? v[i + 1] : dn0;
-        const int cd = code[i];
-        float l = (cd & 1) ? c : fl;
-        float rr = (cd & 2) ? c : fr;
-        float u = (cd & 4) ? c : U;
-        float dd = (cd & 8) ? c : D;
-        if (FACES) {
-          const int pt = part[i];
-          l = (pt & 1) ? __builtin_fmaf(wl[i], fl - c, c) : l;
-          rr = (pt & 2) ? __builtin_fmaf(wr[i], fr - c, c) : rr;
-          u = (pt & 4) ? __builtin_fmaf(wu[i], U - c, c) : u;
-          dd = (pt & 8) ? __builtin_fmaf(wd[i], D - c, c) : dd;
-        }
-        out[i] = __builtin_fmaf(-4.0f, c, ((u + l) + rr) + dd);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float c = v[i];
-        const float U = i > 0 ? v[i - 1] : up0;
-        const float D = i < R - 1 ? v[i + 1] : dn0;
-        // zero-filled shifts at lanes 0 and 63 (halo cells), folded into
-        // the additions as DPP operands
-        out[i] = __builtin_fmaf(-4.0f, c, ((U + jt::lane_shr0(c)) + jt::lane_shl0(c)) + D);
-      }
-    }
-  };
-  if (first) {
-    lap(x, lv);
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      r[i] = lv[i] - r[i];
-      d[i] = r[i] / theta;
-    }
-  }
-  for (int it = 0; it < T; ++it) {
-    lap(d, lv);
-    const float cd = cf.cd[it], cr = cf.cr[it];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      x[i] = x[i] + d[i];
-      r[i] = r[i] + lv[i];
-      d[i] = __builtin_fmaf(cd, d[i], cr * r[i]);
-    }
-  }
-  const bool col_out = lane >= CT_HALO && lane < 64 - CT_HALO && gx < Wc;
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int ty = wave * R + i, gy = gy0 + i;
-    if (col_out && ty >= CT_HALO && ty < CT_EY - CT_HALO && gy < Hc) {
-      const int pos = gy * Wc + gx;
-      xout[pos] = x[i];
-      rout[pos] = r[i];
-      dout[pos] = d[i];
-    }
-  }
+    k_coarse_cheb_tile(nx::jt::ChebArgs a, ChebCoef cf) {
+  nx::jt::cheb_tile<CT_ROWS, CT_WAVES, CT_COLS, FACES, false>(a, cf, (int)blockIdx.x);
 }
 
 namespace nx {
@@ -638,27 +473,32 @@ int launch_coarse_smooth(hipStream_t st, int Wc, int Hc, float* e, const float* 
     if (!ws) return set_error(NX_ERR_ARG, "coarse smoother workspace missing");
     const size_t n = (size_t)Wc * Hc;
     float* set[2][3] = {{ws, ws + n, ws + 2 * n}, {ws + 3 * n, ws + 4 * n, ws + 5 * n}};
-    const dim3 grid((Wc + CT_VX - 1) / CT_VX, (Hc + CT_VY - 1) / CT_VY);
+    constexpr int EX = 64 * CT_COLS, EY = CT_ROWS * CT_WAVES;
+    const int most = nx::jt::cheb_tiles(Wc, Hc, EX, EY, CT_T + 1) <= CT_TILES ? CT_T : CT_T_MANY;
     ChebRecurrence rec(lambda_min);
+    int launches = (iterations + most - 1) / most;
+    // e is the first launch's input and the last one's output: one launch does
+    // only where one tile holds the grid
+    if (launches == 1 && nx::jt::cheb_tiles(Wc, Hc, EX, EY, 1) > 1) launches = 2;
     int done = 0, cur = 0;
-    while (done < iterations) {
-      const int T = iterations - done < CB_T ? iterations - done : CB_T;
-      const bool last = done + T >= iterations;
-      const float* xin = done == 0 ? e : set[cur][0];
-      float** out = set[done == 0 ? 0 : 1 - cur];
+    for (int l = 0; l < launches; ++l) {
+      const int T = (iterations - done + launches - l - 1) / (launches - l);
+      const bool first = l == 0, last = l == launches - 1;
+      float** out = set[first ? 0 : 1 - cur];
       ChebCoef cf{};
-      rec.next(0, T, cf);
+      rec.next(first, T + first, cf);
+      const nx::jt::ChebArgs a{first ? e : set[cur][0], set[cur][1], set[cur][2], rc, mc, faces,
+                               last ? e : out[0], last ? nullptr : out[1], out[2], Wc, Hc, T,
+                               first ? 1 : 0, T + (first ? 1 : 0), rec.theta, nullptr, nullptr,
+                               nullptr};
+      const int grid = nx::jt::cheb_tiles(Wc, Hc, EX, EY, a.halo);
       if (faces)
-        k_coarse_cheb_tile<true><<<grid, 64 * CT_WAVES, 0, st>>>(
-            xin, set[cur][1], set[cur][2], last ? e : out[0], out[1], out[2], rc, mc, faces,
-            Wc, Hc, done, T, rec.theta, cf);
+        k_coarse_cheb_tile<true><<<grid, 64 * CT_WAVES, 0, st>>>(a, cf);
       else
-        k_coarse_cheb_tile<false><<<grid, 64 * CT_WAVES, 0, st>>>(
-            xin, set[cur][1], set[cur][2], last ? e : out[0], out[1], out[2], rc, mc, nullptr,
-            Wc, Hc, done, T, rec.theta, cf);
+        k_coarse_cheb_tile<false><<<grid, 64 * CT_WAVES, 0, st>>>(a, cf);
       if (hipGetLastError() != hipSuccess)
         return set_error(NX_ERR_HIP, "coarse smoother launch failed");
-      cur = done == 0 ? 0 : 1 - cur;
+      cur = first ? 0 : 1 - cur;
       done += T;
     }
   } else if (lambda_min > 0.0f) {
@@ -913,7 +753,7 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
   if (!s->in_step) return fail(NX_ERR_STATE, "nx_smooth_chebyshev outside nx_step_begin/finish");
   if (iterations < 1 || !(lambda_min > 0.0f && lambda_min < 8.0f))
     return fail(NX_ERR_ARG, "iterations >= 1 and 0 < lambda_min < 8 required");
-  const JacobiCfg c = tile ? JacobiCfg{tile[0], tile[1], tile[2], tile[3]} : s->cheb_cfg;
+  JacobiCfg c = tile ? JacobiCfg{tile[0], tile[1], tile[2], tile[3]} : s->cheb_cfg;
   const bool stream = c.seg > 0;
   if (stream ? !stream_cfg_supported(c) : !cheb_cfg_supported(c))
     return fail(NX_ERR_ARG, "unsupported Chebyshev tile");
@@ -933,6 +773,10 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
     NX_HIP(hipMalloc(&s->cheb_red, red_need * sizeof(double)));
     s->cheb_red_cap = red_need;
   }
+  // tiles run even launches, no wider than c.k passes: halos no larger than
+  // their number needs (2048^2, 18 iterations of 15 at most: 10 + 10, not 15 + 5)
+  const int passes = iterations + 2;
+  if (!stream && c.k > 1) c.k = jacobi_even_k(passes, c.k);
   ChebRecurrence rec(lambda_min);
   int done = 0, cur = 0, last_blocks = 0;
   for (bool last = false; !last;) {

@@ -231,11 +231,6 @@ int jacobi_launch_blocks(int W, int H, JacobiCfg c) {
   return jt::axis_tiles(W, 64 * c.cols, c.k) * jt::axis_tiles(H, c.rows * c.waves, c.k);
 }
 
-int cheb_launch_blocks(int W, int H, JacobiCfg c) {
-  const int VX = 64 * c.cols - 2 * c.k, VY = c.rows * c.waves - 2 * c.k;
-  return ((W + VX - 1) / VX) * ((H + VY - 1) / VY);
-}
-
 static hipError_t launch_shape(const float* pin, const float* b, const uint8_t* mask, float* pout,
                                int W, int H, JacobiCfg c, double* red, const int* done,
                                const jt::Project<F32S>& proj, hipStream_t s) {

@@ -13,18 +13,11 @@ namespace jt {
 // its right-hand side and, next to solids, its masks fit in without spills in
 // the sweeps; asked for one step more (8 for 16 cells, 5 for 32) the spills
 // cost more than the waves give (2048^2, (12, 8, 8, 2): 1.96 to 2.27 us per
-// sweep).  A Chebyshev tile of 8 cells per lane takes 83 VGPRs (5 waves, 2
-// blocks of 8 waves); asked for 6 it fits in 80 with one spilled VGPR, and a
-// 3rd block fits.  Its residual variant and the larger tiles would spill
-// heavily, so they stay free.  Tiles of 4 cells per lane ask for 8, so that
-// two blocks of 16 waves fit.
+// sweep).
 template <int CELLS>
 constexpr int jacobi_waves_per_eu() {
   return CELLS <= 8 ? 8 : CELLS <= 16 ? 6 : CELLS <= 32 ? 4 : 2;
 }
-template <int CELLS, bool RES>
-constexpr int cheb_waves_per_eu() { return CELLS <= 4 ? 8 : (CELLS == 8 && !RES ? 6 : 1); }
-
 __device__ __forceinline__ double wave_sum(double v) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;

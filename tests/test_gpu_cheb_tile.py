@@ -1,0 +1,40 @@
+"""The Chebyshev tiles where they can go wrong: grids of exactly one tile, one
+cell more and less, lower or narrower than a tile, launches of one pass to the
+most, with and without solid cells; bitwise against the float32 statement."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+from smoothers import cheb32
+from test_gpu_learned import dev, in_step_sim
+
+from natrix_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("solids", [True, False])
+@pytest.mark.parametrize("W,H,tile,iters", [
+    (128, 128, (20, 8, 8, 2), 18), (129, 127, (20, 8, 8, 2), 19), (127, 129, (9, 8, 8, 2), 20),
+    (300, 40, (20, 8, 8, 2), 40), (17, 300, (12, 8, 8, 2), 25), (261, 263, (16, 4, 16, 2), 34),
+    (128, 64, (2, 4, 16, 2), 3), (140, 70, (8, 8, 8, 1), 16), (131, 133, (7, 4, 8, 2), 6),
+])
+def test_tiles(gpu, rng, W, H, tile, iters, solids):
+    sim = in_step_sim(rng, H, W)
+    solid = sim.download("mask") != 0
+    if not solids:
+        dev(sim, "mask").zero_()
+        solid[:] = False
+    b = rng.normal(size=(H, W)).astype(np.float32)
+    p = rng.normal(size=(H, W)).astype(np.float32)
+    dev(sim, "divergence").copy_(torch.from_numpy(b))
+    dev(sim, "pressure").copy_(torch.from_numpy(p))
+    torch.cuda.synchronize()
+    out = (C.c_double * 2)()
+    _lib.call("nx_smooth_chebyshev", sim._alive(), iters, 0.01, (C.c_int * 4)(*tile), out)
+    got = sim.download("pressure")
+    assert np.array_equal(got, cheb32(p, b, solid, iters, 0.01))
+    assert np.isfinite(out[0])
+    _lib.call("nx_step_finish", sim._alive())
+    sim.destroy()
