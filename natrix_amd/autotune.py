@@ -78,6 +78,32 @@ def lookup(W, H, dtype="f32"):
     return DEFAULT
 
 
+# sides of the grids whose check interval is known, and the sweeps it is made
+# of (nearest cell count; the first of two equally near)
+CHECK_UNITS = ((1024, 10), (256, 12), (512, 16))
+
+
+def check_interval(W, H, check_every):
+    """Sweeps between two residual checks of a tolerance solve on a tuned
+    tile: `check_every`, rounded up to whole units of the grid.  Where a solve
+    stops is part of its result, so the unit belongs to the grid and not to
+    the table's tile, whose sweeps per launch a retune may change."""
+    _, unit = min(CHECK_UNITS, key=lambda t: abs(t[0] * t[0] - W * H))
+    return -(-check_every // unit) * unit
+
+
+def solve_sweeps(W, H, k, check_every):
+    """Sweeps per launch, at most the tuned tile's k, with which a tolerance
+    solve checks its residual every check_interval() sweeps: the most that
+    divide the interval and, rounded up to by nx_update, still give it (the
+    grid's unit is one such whenever k reaches it)."""
+    chunk = check_interval(W, H, check_every)
+    for d in range(k, 0, -1):
+        if chunk % d == 0 and -(-check_every // d) * d == chunk:
+            return d
+    return k
+
+
 SMOOTHER_DEFAULT = (8, 4, 8, 2)
 
 

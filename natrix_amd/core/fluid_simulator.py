@@ -125,7 +125,8 @@ class FluidSimulator:
         self.check_every = 256
         self.correction_sweeps = 8
         from ..autotune import lookup, lookup_smoother
-        self.jacobi_tile = lookup(self._width, self._height, storage)
+        self._jacobi_tile = lookup(self._width, self._height, storage)
+        self._tile_tuned = True
         if storage == "f32":
             self.smoother_tile = lookup_smoother(self._width, self._height)
         self._dye_speed = 500.0
@@ -219,6 +220,20 @@ class FluidSimulator:
         self._bc_mode = int(value)
 
     @property
+    def jacobi_tile(self):
+        """(sweeps per launch, rows, waves, cols[, seg]) of the Jacobi
+        launches: the tuned tile of the grid until one is set.  A tolerance
+        solve checks its residual after whole launches: on a tile set here
+        every ceil(check_every / k) of them, on the tuned tile every
+        autotune.check_interval() sweeps, whatever the table's k."""
+        return self._jacobi_tile
+
+    @jacobi_tile.setter
+    def jacobi_tile(self, tile):
+        self._jacobi_tile = tile
+        self._tile_tuned = False
+
+    @property
     def use_graph(self):
         return self._use_graph
 
@@ -228,7 +243,8 @@ class FluidSimulator:
         _lib.call("nx_set_graph", self._h, int(self._use_graph))
 
     # ------------------------------------------------------------ internals
-    def _push_params(self):
+    def _push_params(self, solve=False):
+        """solve: the caller runs tolerance solves (nx_solve) inside the step."""
         p = self._prm
         p.speed = self._speed
         p.dissipation = self._dissipation
@@ -248,6 +264,9 @@ class FluidSimulator:
         p.tol = float(self.tol)
         p.max_iters = int(self.max_iters)
         p.check_every = int(self.check_every)
+        if self._tile_tuned and (solve or p.tol > 0) and p.check_every > 0:
+            from ..autotune import solve_sweeps
+            p.jacobi_k = solve_sweeps(self._width, self._height, p.jacobi_k, p.check_every)
         p.correction_sweeps = int(self.correction_sweeps)
         _lib.call("nx_set_params", self._h, C.byref(p))
 

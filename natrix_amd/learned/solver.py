@@ -359,7 +359,7 @@ def solve_step(sim, guess, dt, tol=1e-4, inner_tol=0.1, smooth=72, max_cycles=6,
         lmin = guess.fine_lmin(sim.width, sim.height) if guess is not None else 0.0
     else:
         lmin = float(fine_lmin)
-    sim._push_params()
+    sim._push_params(solve=True)
     _lib.call("nx_step_begin", sim._alive(), float(dt))
     _lib.call("nx_refine_begin", sim._alive())
     stream = torch.cuda.ExternalStream(sim.stream_handle())
