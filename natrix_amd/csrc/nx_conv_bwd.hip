@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(256)
            uint16_t* __restrict__ dz, const float* __restrict__ w,
            const float* __restrict__ dout, float* __restrict__ part, long long rows, int C,
            long long rows_per_block) {
-  extern __shared__ float acc[];  // [groups][C]
+  extern __shared__ float acc[];  // [groups][C], groups > 1
   const int cg = C / V;           // channel groups of a row
   const int gang = cg < 256 ? cg : 256;
   const int groups = 256 / gang;  // rows a block works on at once
@@ -133,15 +133,23 @@ __global__ void __launch_bounds__(256)
             dz[at] = ov[0];
         }
       }
+      // a row as wide as the block: the thread's sum is the block's
 #pragma unroll
-      for (int j = 0; j < V; ++j) acc[g * C + c * V + j] = s[j];
+      for (int j = 0; j < V; ++j) {
+        if (groups > 1)
+          acc[g * C + c * V + j] = s[j];
+        else
+          part[(long long)blockIdx.x * width + c * V + j] = s[j];
+      }
     }
   }
-  __syncthreads();
-  for (int c = threadIdx.x; c < C; c += 256) {
-    float s = 0.0f;
-    for (int q = 0; q < groups; ++q) s += acc[q * C + c];
-    part[(long long)blockIdx.x * width + c] = s;
+  if (groups > 1) {
+    __syncthreads();
+    for (int c = threadIdx.x; c < C; c += 256) {
+      float s = 0.0f;
+      for (int q = 0; q < groups; ++q) s += acc[q * C + c];
+      part[(long long)blockIdx.x * width + c] = s;
+    }
   }
   if (MODE == SUM_HEAD) {
     __shared__ float d[1024];
@@ -202,8 +210,7 @@ int launch_rows(const uint16_t* a, const uint16_t* dy, uint16_t* dz, const float
                    (((uintptr_t)a | (uintptr_t)dy | (uintptr_t)dz) & 15) == 0;
   const int cg = vec ? C / 8 : C;
   const int groups = cg < 256 ? 256 / cg : 1;
-  const size_t lds = (size_t)groups * C * sizeof(float);
-  if (lds > 61440) return nx::set_error(NX_ERR_ARG, "row pass: too many channels");
+  const size_t lds = groups > 1 ? (size_t)groups * C * sizeof(float) : 0;  // at most 8 KiB
   if (vec)
     k_rows<MODE, 8><<<(unsigned)blocks, 256, lds, s>>>(a, dy, dz, w, dout, part, rows, C, per);
   else

@@ -116,6 +116,35 @@ def test_head_backward(gpu, pixels, c):
         pixels * 2.0 ** -24 * float(dout.double().abs().sum())
 
 
+@pytest.mark.parametrize("rows,c", [(3, 1032), (70, 2048), (130, 2056), (3, 15361), (65, 20000)])
+def test_row_passes_of_many_channels(gpu, rows, c):
+    """Rows as wide as a block and wider (256 threads of one or eight channels),
+    beyond what a block's LDS would hold."""
+    g = torch.Generator().manual_seed(rows + c)
+    y = torch.randn(rows, c, generator=g).to(BF)
+    dy = torch.randn(rows, c, generator=g).to(BF)
+    w, dout = torch.randn(c, generator=g), torch.randn(rows, generator=g)
+    yd, dyd, wd, dd = y.cuda(), dy.cuda(), w.cuda(), dout.cuda()
+    dz = torch.full_like(dyd, float("nan"))
+    db, dwb = (torch.full((c + i,), float("nan"), device="cuda") for i in (0, 1))
+    work = torch.full((1024 * (c + 1),), float("nan"), device="cuda")
+    _lib.call("nx_relu_bwd_colsum", _p(yd), _p(dyd), _p(dz), _p(db), _p(work), rows, c, _s())
+    want = torch.where(y > 0, dy, torch.zeros_like(dy))
+    assert torch.equal(dz.cpu(), want)
+    unit = rows * 2.0 ** -24
+    assert bool(((db.double().cpu() - want.double().sum(0)).abs() <=
+                 unit * want.double().abs().sum(0)).all())
+    _lib.call("nx_colsum", _p(dyd), _p(db), _p(work), rows, c, _s())
+    assert bool(((db.double().cpu() - dy.double().sum(0)).abs() <=
+                 unit * dy.double().abs().sum(0)).all())
+    _lib.call("nx_head_bwd", _p(yd), _p(wd), _p(dd), _p(dz), _p(dwb), _p(work), rows, c, _s())
+    assert torch.equal(dz.cpu(), (dout[:, None] * w).to(BF))
+    terms = dout.double()[:, None] * y.double()
+    assert bool(((dwb[:c].double().cpu() - terms.sum(0)).abs() <=
+                 (rows + 1) * 2.0 ** -24 * terms.abs().sum(0)).all())
+    assert abs(float(dwb[c]) - float(dout.double().sum())) <= unit * float(dout.double().abs().sum())
+
+
 @pytest.mark.parametrize("n,h,w,ca,cb", [(1, 2, 2, 8, 16), (2, 6, 10, 64, 32), (1, 4, 2, 5, 3),
                                          (3, 8, 4, 24, 12)])
 def test_movers_wide_and_single(gpu, n, h, w, ca, cb):
