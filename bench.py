@@ -150,7 +150,7 @@ def cheb_launch_plan(iterations, k):
     (the library's launch loop)."""
     plan, done = [], 0
     while True:
-        setup = 1 if done == 0 else 0
+        setup = 1 if not plan else 0
         last = setup + (iterations - done) + 1 <= k
         kk = setup + (iterations - done) + 1 if last else k
         its = kk - setup - (1 if last else 0)

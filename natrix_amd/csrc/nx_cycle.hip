@@ -776,11 +776,10 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
   // tiles run even launches, no wider than c.k passes: halos no larger than
   // their number needs (2048^2, 18 iterations of 15 at most: 10 + 10, not 15 + 5)
   const int passes = iterations + 2;
-  if (!stream && c.k > 1) c.k = jacobi_even_k(passes, c.k);
+  if (!stream) c.k = jacobi_even_k(passes, c.k);
   ChebRecurrence rec(lambda_min);
-  int done = 0, cur = 0, last_blocks = 0;
+  int done = 0, cur = 0, last_blocks = 0, setup = 1;
   for (bool last = false; !last;) {
-    const int setup = done == 0 ? 1 : 0;
     JacobiCfg cc = c;
     last = setup + (iterations - done) + 1 <= c.k;
     cc.k = last ? setup + (iterations - done) + 1 : c.k;
@@ -811,6 +810,7 @@ static int smooth_cheb_impl(nx_sim* s, int iterations, float lambda_min, const i
     s->pcur ^= 1;
     cur ^= 1;
     done += its;
+    setup = 0;  // one launch's, also where it had no pass left to iterate (k = 1)
   }
   s->step_sweeps += iterations;
   // the residual and the line-search step land in pinned host memory,

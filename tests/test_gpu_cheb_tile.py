@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 import torch
-from smoothers import cheb32
+from smoothers import cheb32, lap
 from test_gpu_learned import dev, in_step_sim
 
 from natrix_amd import _lib
@@ -38,3 +38,36 @@ def test_tiles(gpu, rng, W, H, tile, iters, solids):
     assert np.isfinite(out[0])
     _lib.call("nx_step_finish", sim._alive())
     sim.destroy()
+
+
+@pytest.mark.parametrize("W,H,iters", [(140, 70, 5), (64, 33, 1), (17, 300, 4)])
+@pytest.mark.parametrize("tile", [(1, 8, 8, 2, 0), (1, 4, 16, 1, 0), (1, 4, 8, 2, 24)])
+def test_one_pass_a_launch(gpu, rng, W, H, iters, tile):
+    """k = 1, tile and streaming: the first launch only sets up, each of the next
+    runs one iteration, the last only takes the residual."""
+    sim = in_step_sim(rng, H, W)
+    solid = sim.download("mask") != 0
+    b = rng.normal(size=(H, W)).astype(np.float32)
+    p = rng.normal(size=(H, W)).astype(np.float32)
+    dev(sim, "divergence").copy_(torch.from_numpy(b))
+    dev(sim, "pressure").copy_(torch.from_numpy(p))
+    torch.cuda.synchronize()
+    sim.smoother_tile = tile if tile[4] else tile[:4]
+    sim.set_timing(True)
+    sim.collect_timing()
+    out = (C.c_double * 2)()
+    _lib.call("nx_smooth_chebyshev", sim._alive(), iters, 0.01, None, out)
+    assert sim.collect_timing()["chebyshev"][1] == iters + 2
+    got = sim.download("pressure")
+    assert np.array_equal(got, cheb32(p, b, solid, iters, 0.01))
+    _check_residual(out[0], got, b, solid)
+    _lib.call("nx_step_finish", sim._alive())
+    sim.destroy()
+
+
+def _check_residual(rel, p, b, solid):
+    r = (b.astype(np.float64) - lap(p.astype(np.float64), solid))[~solid]
+    bf = b.astype(np.float64)[~solid]
+    n = r.size
+    want = np.sqrt((np.sum(r * r) - np.sum(r) ** 2 / n) / (np.sum(bf * bf) - np.sum(bf) ** 2 / n))
+    assert abs(rel - want) <= 1e-9 * want
