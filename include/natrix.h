@@ -200,8 +200,8 @@ int nx_coarse_smooth(nx_sim* sim, int Wc, int Hc, float* e, const float* rc,
  * problem (no reference counterpart): (L e)_I = sum over the faces of I of
  * w (e_J - e_I) with the weights of nx_restrict_residual_faces (spectrum
  * of -L in [0, 8]); a neighbour across a face of weight w enters as the
- * centre (w = 0), itself (w = 1) or fma(w, e_J - e_I, e_I), summed in the
- * plain kernel's order */
+ * centre (w = 0), itself (w = 1, and any weight outside [0, 1]) or
+ * fma(w, e_J - e_I, e_I), summed in the plain kernel's order */
 int nx_coarse_smooth_faces(nx_sim* sim, int Wc, int Hc, float* e, const float* rc,
                            const uint8_t* coarse_mask, const float* faces, int iterations,
                            float lambda_min);

@@ -164,6 +164,17 @@ __device__ __forceinline__ void cheb_tile(const ChebArgs& a, const ChebCoef& cf,
     for (int i = 0; i < FR; ++i) load_row(a.faces, gy0 + i, fe[i]);
 #pragma unroll
     for (int i = 0; i <= FR; ++i) load_row(south, gy0 - 1 + i, fs[i]);
+    // a weight outside [0, 1] is an open face
+    auto clean = [](float& w) { w = w >= 0.0f && w < 1.0f ? w : 1.0f; };
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) {
+      clean(fs[0][c]);
+#pragma unroll
+      for (int i = 0; i < FR; ++i) {
+        clean(fe[i][c]);
+        clean(fs[i + 1][c]);
+      }
+    }
     bool any = false;
     auto inner = [](float w) { return w > 0.0f && w < 1.0f; };
 #pragma unroll

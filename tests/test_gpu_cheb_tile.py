@@ -71,3 +71,31 @@ def _check_residual(rel, p, b, solid):
     n = r.size
     want = np.sqrt((np.sum(r * r) - np.sum(r) ** 2 / n) / (np.sum(bf * bf) - np.sum(bf) ** 2 / n))
     assert abs(rel - want) <= 1e-9 * want
+
+
+@pytest.mark.parametrize("partial", [True, False])
+@pytest.mark.parametrize("Wc,Hc,iters", [(128, 128, 5), (100, 72, 40), (7, 60, 12)])
+def test_face_weights_outside_the_unit_interval_are_open(gpu, rng, Wc, Hc, iters, partial):
+    """Whether or not the wave holds partial faces, whose form of the sweep
+    multiplies by the weight."""
+    sim = in_step_sim(rng, 64, 64)
+    kinds = [0.0, 0.25, 0.75, 1.0] if partial else [0.0, 1.0, 1.0]
+    plain = rng.choice(kinds, size=(2, Hc, Wc)).astype(np.float32)
+    odd = plain.copy()
+    at = rng.random(plain.shape) < 0.2
+    odd[at] = rng.choice([1.5, -0.5, np.nan, np.inf], size=int(at.sum()))
+    plain[at] = 1.0
+    e0, rc = (rng.normal(size=(Hc, Wc)).astype(np.float32) for _ in range(2))
+    mc = torch.zeros((Hc, Wc), dtype=torch.uint8, device="cuda")
+    got = []
+    for faces in (plain, odd):
+        e, r, f = (torch.from_numpy(a).cuda() for a in (e0, rc, faces))
+        torch.cuda.synchronize()
+        _lib.call("nx_coarse_smooth_faces", sim._alive(), Wc, Hc,
+                  *(C.c_void_p(t.data_ptr()) for t in (e, r, mc, f)), iters, 0.05)
+        sim.synchronize()
+        got.append(e.cpu().numpy())
+    assert np.isfinite(got[0]).all()
+    assert np.array_equal(got[0], got[1])
+    _lib.call("nx_step_finish", sim._alive())
+    sim.destroy()
