@@ -1,5 +1,6 @@
-// 3x3 convolution over many pixels (gfx950): the training path's forward and
-// input gradient, where one launch has enough tiles to fill the chip.
+// 3x3 convolution staged in LDS (gfx950): the training path's forward and input
+// gradient, wherever no split of K and no tiled weights are asked for and the
+// image is more than a few pixels (conv3x3_lds has the line).
 // Layouts and arithmetic as in nx_unet.hip: NHWC bfloat16 activations, KRSC
 // bfloat16 weights, and for every output the chain of v_mfma_f32_32x32x16_bf16
 // over the K steps in order (16 channels of one tap, taps outermost), so the
@@ -196,6 +197,14 @@ bool conv3x3_lds(const uint16_t* x, const uint16_t* w, const float* bias, uint16
                  int h, int wd, int cin, int cout, int relu, hipStream_t s, hipError_t* err) {
   if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) != 0) return false;
   if ((long long)n * ((h + 7) / 8) * ((wd + 15) / 16) > 0x7FFFFFFF) return false;
+  // A few pixels: k_conv3x3, whose waves take 32 or 64 of them, starts on its
+  // first fragments while a block here still stages the weights of 128 channels
+  // or more.  us with k_conv3x3 / here, at 16, 48 and 64 pixels: 128 -> 128
+  // channels 25.4 / 28.6, 30.1 / 28.9, 33.1 / 28.8; 256 -> 256 45.0 / 54.5,
+  // 50.7 / 54.6, 54.6 / 54.7.  With 32 to 96 channels (64 -> 64: 13.3 / 12.3 at
+  // one pixel) and with 192 and 384 (384 -> 128: 62 / 50) staging wins from one
+  // pixel on.
+  if ((cin == 128 || cin == 256) && (long long)n * h * wd * 3 <= cin) return false;
   const bool n2 = cout % 64 == 0, n4 = cout % 128 == 0;
 #define NX_CONV(CPS, NT, WN, CH) \
   return *err = launch<CPS, NT, WN, CH>(x, w, bias, y, n, h, wd, cout, relu, s), true

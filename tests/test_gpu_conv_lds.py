@@ -57,6 +57,13 @@ def test_conv_lds(gpu, n, h, w, ci, co, relu):
     assert bool((err <= 9 * ci * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs()).all())
 
 
+@pytest.mark.parametrize("n,h,w,ci,co", [(1, 6, 7, 128, 128), (1, 1, 43, 128, 64),
+                                         (5, 1, 17, 256, 256), (2, 1, 43, 256, 128)])
+def test_either_side_of_the_pixel_line(gpu, n, h, w, ci, co):
+    """The last image that is not staged and the first that is (cin / 3 pixels)."""
+    test_conv_lds(gpu, n, h, w, ci, co, 1)
+
+
 def test_conv_without_bias_and_infinities(gpu):
     """No bias (the input gradient's call); an infinite pixel reaches its 3 x 3
     neighbourhood and nothing else."""
