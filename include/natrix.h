@@ -263,6 +263,8 @@ int nx_step_finish(nx_sim* sim);
  * nx_update calls with the same dt and parameters (on = 1); steps of a few
  * launches, which cost less enqueued than replayed, are enqueued. */
 int nx_set_graph(nx_sim* sim, int on);
+/* steps replayed from a graph since the simulator was made */
+int nx_graph_replays(nx_sim* sim, long long* out);
 
 /* ---- per-stage entry points (one reference shader each), operating on the
  *      simulator's current buffers in the reference's slot semantics ---- */
@@ -343,6 +345,7 @@ int nx_batch_add_triangle_obstacle(nx_batch* b, int scene, float x1, float y1, f
 int nx_batch_set_step_splats(nx_batch* b, const float* rec, int n);
 int nx_batch_update(nx_batch* b, float dt);
 int nx_batch_set_graph(nx_batch* b, int on);
+int nx_batch_graph_replays(nx_batch* b, long long* out);
 int nx_batch_jacobi_blocked(nx_batch* b, int sweeps, int k, int rows, int waves,
                             int cols);
 int nx_batch_upload(nx_batch* b, int scene, int field, const void* src,

@@ -97,6 +97,7 @@ SIGNATURES = {
     "nx_set_obstacle_map": [_P, C.POINTER(C.c_uint8)],
     "nx_update": [_P, _F],
     "nx_set_graph": [_P, _I],
+    "nx_graph_replays": [_P, C.POINTER(C.c_longlong)],
     "nx_stage_boundaries": [_P],
     "nx_stage_advect": [_P, _F],
     "nx_stage_curl": [_P],
@@ -129,6 +130,7 @@ SIGNATURES = {
     "nx_batch_set_step_splats": [_P, C.POINTER(_F), _I],
     "nx_batch_update": [_P, _F],
     "nx_batch_set_graph": [_P, _I],
+    "nx_batch_graph_replays": [_P, C.POINTER(C.c_longlong)],
     "nx_batch_jacobi_blocked": [_P, _I, _I, _I, _I, _I],
     "nx_batch_upload": [_P, _I, _I, _P, _SZ],
     "nx_batch_download": [_P, _I, _I, _P, _SZ],

@@ -106,12 +106,21 @@ class BatchedScenes:
 
     @property
     def use_graph(self):
+        """As FluidSimulator.use_graph: steps of ten launches and more are
+        captured and replayed, shorter ones enqueued."""
         return getattr(self, "_graph", False)
 
     @use_graph.setter
     def use_graph(self, on):
         self._graph = bool(on)
         _lib.call("nx_batch_set_graph", self._alive(), int(self._graph))
+
+    @property
+    def graph_replays(self):
+        """Steps replayed from a graph so far."""
+        n = C.c_longlong()
+        _lib.call("nx_batch_graph_replays", self._alive(), C.byref(n))
+        return n.value
 
     def add_circle_obstacle(self, scene, position, radius, static=False):
         """FluidSimulator.add_circle_obstacle for one scene (this step)."""

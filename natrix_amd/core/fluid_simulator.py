@@ -235,12 +235,23 @@ class FluidSimulator:
 
     @property
     def use_graph(self):
+        """Capture fixed-iteration steps into HIP graphs, replayed by later
+        updates with the same dt and parameters.  Steps of fewer than ten
+        launches are enqueued instead, which costs less and gives the same
+        results; graph_replays tells which happened."""
         return self._use_graph
 
     @use_graph.setter
     def use_graph(self, on):
         self._use_graph = bool(on)
         _lib.call("nx_set_graph", self._h, int(self._use_graph))
+
+    @property
+    def graph_replays(self):
+        """Steps replayed from a graph so far."""
+        n = C.c_longlong()
+        _lib.call("nx_graph_replays", self._alive(), C.byref(n))
+        return n.value
 
     # ------------------------------------------------------------ internals
     def _push_params(self, solve=False):

@@ -878,6 +878,7 @@ int nx_update(nx_sim* s, float dt) {
     s->graph_prm[par] = P;
   }
   NX_HIP(hipGraphLaunch(s->graph[par], s->stream));
+  ++s->graph_replays;
   // replay the index bookkeeping of step_fused_enqueue
   const int sweeps_tb = P.iterations - 1;
   int pc = 0, rem = sweeps_tb;
@@ -989,6 +990,12 @@ int nx_step_finish(nx_sim* s) {
     s->dcur ^= 1;
   }
   s->in_step = false;
+  return NX_OK;
+}
+
+int nx_graph_replays(nx_sim* s, long long* out) {
+  if (!s || !out) return fail(NX_ERR_ARG, "null argument");
+  *out = s->graph_replays;
   return NX_OK;
 }
 

@@ -273,6 +273,7 @@ struct nx_batch {
   hipGraphExec_t graph[8] = {};
   float graph_dt[8] = {};
   nx_params graph_prm[8];
+  long long graph_replays = 0;
 };
 
 extern "C" int nx_batch_destroy(nx_batch* b);
@@ -669,6 +670,7 @@ int nx_batch_update(nx_batch* b, float dt) {
     b->graph_prm[par] = P;
   }
   NXB_HIP(hipGraphLaunch(b->graph[par], b->stream));
+  ++b->graph_replays;
   int pcn = 0, rem = P.iterations - 1;
   while (rem > 0) {
     rem -= std::min(rem, P.jacobi_k);
@@ -678,6 +680,12 @@ int nx_batch_update(nx_batch* b, float dt) {
   b->vcur ^= 1;
   b->mcur ^= 1;
   if (dye) b->dcur ^= 1;
+  return NX_OK;
+}
+
+int nx_batch_graph_replays(nx_batch* b, long long* out) {
+  if (!b || !out) return bfail(NX_ERR_ARG, "null argument");
+  *out = b->graph_replays;
   return NX_OK;
 }
 

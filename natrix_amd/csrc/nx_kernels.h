@@ -80,10 +80,13 @@ struct JacobiCfg {
   int cols;     // columns per lane
   int seg = 0;  // > 0: streaming kernel, output rows per workgroup segment
 };
-// A captured step is replayed only from this many launches on: a launch costs the
-// host 2.7 us, a replay 15 us and 1 us a node (256^2, 40 sweeps, 4 launches: 13.7
-// us a step enqueued, 21.9 replayed, three simulators in turn; 1024^2, 5
-// launches: 66.7 and 68.5), and the results are the same.
+// A captured step is replayed only from this many launches on; the results are the
+// same.  A launch costs the host 3 us, a replay 15 us and 1 to 2 us a node.
+// us a step enqueued / replayed, three simulators in turn, and alone (waited for):
+//   launches     3            6            8            9            10           13
+//   128^2   10.3 / 18.1  18.1 / 20.4  25.3 / 22.4  26.7 / 23.5  29.3 / 25.7  47.3 / 32.6
+//   512^2   20.8 / 20.8  19.8 / 20.7  25.7 / 26.0  28.4 / 28.9  31.3 / 31.7  45.3 / 40.1
+//   alone   38.6 / 45.4  55.6 / 60.9  71.6 / 74.1  78.9 / 80.6  86.0 / 87.2  107  / 106
 constexpr int GRAPH_MIN_LAUNCHES = 10;
 
 // sweeps per launch that spread `sweeps` evenly over ceil(sweeps / k) launches

@@ -96,6 +96,7 @@ struct nx_sim {
   hipGraphExec_t graph[8] = {};
   float graph_dt[8] = {};
   nx_params graph_prm[8];
+  long long graph_replays = 0;
 };
 
 inline int get_event(nx_sim* s, hipEvent_t* ev) {
