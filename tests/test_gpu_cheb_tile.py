@@ -65,6 +65,25 @@ def test_one_pass_a_launch(gpu, rng, W, H, iters, tile):
     sim.destroy()
 
 
+@pytest.mark.parametrize("W,H,tile,iters", [
+    (129, 127, (20, 8, 8, 2), 19), (300, 40, (20, 8, 8, 2), 40), (261, 263, (16, 4, 16, 2), 34),
+    (128, 64, (2, 4, 16, 2), 3), (140, 70, (8, 8, 8, 1), 16), (131, 133, (7, 4, 8, 2), 6),
+    (200, 150, (3, 8, 16, 1), 1)])
+def test_residual_of_several_tiles(gpu, rng, W, H, tile, iters):
+    """The last launch's residual, whose tiles shrink by one stencil less than
+    their passes: every fluid cell in one record."""
+    sim = in_step_sim(rng, H, W)
+    solid = sim.download("mask") != 0
+    b = rng.normal(size=(H, W)).astype(np.float32)
+    dev(sim, "divergence").copy_(torch.from_numpy(b))
+    torch.cuda.synchronize()
+    out = (C.c_double * 2)()
+    _lib.call("nx_smooth_chebyshev", sim._alive(), iters, 0.01, (C.c_int * 4)(*tile), out)
+    _check_residual(out[0], sim.download("pressure"), b, solid)
+    _lib.call("nx_step_finish", sim._alive())
+    sim.destroy()
+
+
 def _check_residual(rel, p, b, solid):
     r = (b.astype(np.float64) - lap(p.astype(np.float64), solid))[~solid]
     bf = b.astype(np.float64)[~solid]

@@ -82,3 +82,35 @@ def test_even_launches_reach_the_sweep_count(gpu):
         sim.jacobi_blocked(n, 24, 8, 8, 1)
         assert np.array_equal(sim.download("pressure"), F.jacobi(p, b, obs, n)), n
     sim.destroy()
+
+
+@pytest.mark.parametrize("tile", [(8, 8, 8, 1), (12, 4, 16, 1), (8, 4, 8, 2), (20, 8, 8, 2)])
+def test_residual_records_of_several_tiles(gpu, tile):
+    """A tolerance solve on several uneven tiles with solids stops at the check,
+    every ceil(60 / k) k sweeps, at which the oracle's residual meets the
+    tolerance: each cell is in one tile's record."""
+    w, h, tol = 150, 90, 1.5e-3
+    rng = np.random.default_rng(8)
+    y, x = np.mgrid[0:h, 0:w]
+    solid = (x - 60) ** 2 + (y - 40) ** 2 <= 100
+    solid[:, 100] = rng.random(h) < 0.5
+    sim = FluidSimulator(w, h, bc_mode="free_slip")
+    sim.vorticity, sim.viscosity = 0.3, 0.0
+    sim.jacobi_tile, sim.tol, sim.check_every = tile, tol, 60
+    sim.set_obstacle_map(solid)
+    sim.upload("velocity", rng.uniform(-0.5, 0.5, (h, w, 2)).astype(np.float32))
+    obs = F.obstacles_from_mask(sim.download("mask"))
+    sim.update(1 / 60)
+    st, got, b = sim.stats(), sim.download("pressure"), sim.download("divergence")
+    sim.destroy()
+    chunk = -(-60 // tile[0]) * tile[0]
+    p, sweeps, checks = (np.float32(0) - b) * np.float32(0.25), 1, 0
+    while checks < 400:
+        before = F.jacobi(p, b, obs, chunk - 1)
+        p = F.jacobi(before, b, obs, 1)
+        sweeps, checks = sweeps + chunk, checks + 1
+        if F.relative_residual(before, b, obs) <= tol and F.relative_residual(p, b, obs) <= tol:
+            break
+    assert st["converged"] and st["sweeps"] == sweeps and checks > 3
+    assert np.array_equal(got, p)
+    assert abs(st["residual"] - F.relative_residual(p, b, obs)) <= 1e-9
