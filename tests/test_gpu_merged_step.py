@@ -6,6 +6,7 @@ import pytest
 
 from natrix_amd import FluidSimulator
 from oracle import fluid as F
+from oracle import mixed as M
 
 pytestmark = pytest.mark.gpu
 
@@ -98,3 +99,25 @@ def test_splats_far_and_near_a_zero_weight(gpu):
     ref, _ = F.gaussian_splat(u, None, [tuple(np.float32(v) for v in s) for s in splats])
     assert np.array_equal(sim.download("velocity").view(np.uint32), ref.view(np.uint32))
     sim.destroy()
+
+
+@pytest.mark.parametrize("storage", ["bf16", "f16"])
+@pytest.mark.parametrize("iters,corr", [(1, 8), (1, 0), (2, 0), (2, 16), (13, 3)])
+def test_merged_reduced_storage_is_the_replay(gpu, storage, iters, corr):
+    """One iteration leaves the correction launch alone, which also projects;
+    no correction sweeps, and the most."""
+    w, h = 150, 90
+    sims, u, solid = _pair(w, h, storage, "inflow", 0.0, iters, 21)
+    u = M.rounder(storage)(u)
+    prm = F.Params(vorticity=0.3, viscosity=0.0, iterations=iters, bc_mode=F.BC_INFLOW)
+    v, p, p32, b, _ = M.step_mixed(u, np.zeros((h, w, 2), np.float32), np.float32(1 / 60), prm,
+                                   storage, 6, corr, persistent=solid)
+    for sim in sims:
+        sim.jacobi_tile = (6, 8, 8, 2)
+        sim.correction_sweeps = corr
+        sim.upload("velocity", u)
+        sim.update(1 / 60)
+        assert np.array_equal(sim.download("velocity"), v)
+        assert np.array_equal(sim.download("pressure32"), p32)
+        assert np.array_equal(sim.download("divergence"), b)
+        sim.destroy()
