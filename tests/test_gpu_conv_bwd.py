@@ -171,3 +171,14 @@ def test_movers_wide_and_single(gpu, n, h, w, ca, cb):
     up = (((e[:, :, 0, :, 0] + e[:, :, 0, :, 1]) + e[:, :, 1, :, 0]) + e[:, :, 1, :, 1]).to(BF)
     pool = (up.float() * 0.25).to(BF)
     assert torch.equal(xg.grad.cpu(), pool.repeat_interleave(2, 1).repeat_interleave(2, 2))
+
+
+def test_relu_gradient_alone(gpu):
+    """nx_relu_bwd, the gradient without the bias sums that the layers take with it."""
+    g = torch.Generator().manual_seed(2)
+    y = torch.randn(3, 257, generator=g).to(BF).relu()
+    dy = torch.randn(3, 257, generator=g).to(BF)
+    yd, dyd = y.cuda(), dy.cuda()
+    dz = torch.full_like(dyd, float("nan"))
+    _lib.call("nx_relu_bwd", _p(yd), _p(dyd), _p(dz), dy.numel(), _s())
+    assert torch.equal(dz.cpu(), torch.where(y > 0, dy, torch.zeros_like(dy)))
