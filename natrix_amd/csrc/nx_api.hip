@@ -96,11 +96,14 @@ static void invalidate_graphs(nx_sim* s) {
 }
 
 // `sweeps` temporal-blocked sweeps starting from p[pcur], in as many launches
-// as c.k sweeps each take, of equal length: the halo a launch recomputes grows
-// with its sweeps, so 25 + 24 costs less than 28 + 21.  u != nullptr (tile
-// shapes): the last launch projects u in place and writes the next step's mask.
+// as c.k sweeps each take.  Tile launches are of equal length: the halo they
+// recompute grows with their sweeps, so 25 + 24 costs less than 28 + 21.
+// Streaming launches have no such halo, and even ones may use float2 accesses
+// (1000 x 700, 49 sweeps of 8 at most: 178 us, evened out to 7 199 us): they
+// take c.k.  u != nullptr (tile shapes): the last launch projects u in place and
+// writes the next step's mask.
 int nx::run_jacobi_tb(nx_sim* s, int sweeps, JacobiCfg c, float2* u) {
-  c.k = jacobi_even_k(sweeps, c.k);
+  if (c.seg == 0) c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;
