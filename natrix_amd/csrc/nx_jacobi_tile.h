@@ -284,6 +284,13 @@ __device__ __forceinline__ void jacobi_tb_tile(
     }
   };
 
+  constexpr bool SMALL = ROWS * COLS <= 8;
+  // Small strips of few rows keep their masks as conditions, one lane mask in
+  // scalar registers each (20 pairs for 4 x 2 cells), which saves an extraction
+  // per side and the vector registers; 8 rows' 26 pairs spill (1024^2 bf16, 100
+  // iterations: (10, 4, 16, 2) with obstacles 138.6 to 135.7 us a step, (10, 8, 8,
+  // 1) without any 132 to 134.5).
+  constexpr bool CONDS = SMALL && ROWS <= 4;
   double sr = 0.0, srr = 0.0;
   // The passes of one wave.  XE, the x neighbours at the grid's sides: 0 none
   // (a tile away from them), 1 the tile's first and last column, 2 any column
@@ -305,7 +312,21 @@ __device__ __forceinline__ void jacobi_tb_tile(
     // cells left and right of the lane's columns, 2 per row
     constexpr int MR = SP == 1 ? ROWS + 2 : 1, OW = SP == 1 ? (2 * ROWS + 31) / 32 : 1;
     uint32_t msk[MR][COLS], outer[OW];
-    if (SP == 1) {
+    bool fl[MR][COLS], fo[MR][2];
+    if (SP == 1 && CONDS) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) {
+        const int l = ilane_from_left((int)solid(r, COLS - 1));
+        const int q = ilane_from_right((int)solid(r, 0));
+        fo[SP == 1 ? r : 0][0] = gx0 == 0 || l != 0;
+        fo[SP == 1 ? r : 0][1] = right < COLS || q != 0;
+      }
+#pragma unroll
+      for (int r = -1; r <= ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c)
+          fl[SP == 1 ? r + 1 : 0][c] = c > right || r > last || solid(r, c) != 0;
+    } else if (SP == 1) {
 #pragma unroll
       for (int q = 0; q < OW; ++q) outer[q] = 0;
 #pragma unroll
@@ -337,7 +358,14 @@ __device__ __forceinline__ void jacobi_tb_tile(
       x2 = c < COLS - 1 ? v[r][c < COLS - 1 ? c + 1 : c] : lane_shl0(v[r][0]);
       y1 = r > 0 ? v[r > 0 ? r - 1 : 0][c] : prev[c];
       y2 = r < ROWS - 1 ? v[r < ROWS - 1 ? r + 1 : r][c] : above[c];
-      if (SP == 1) {
+      if (SP == 1 && CONDS) {
+        const int m = SP == 1 ? r : 0;
+        const int m1 = SP == 1 ? r + 1 : 0, m2 = SP == 1 ? r + 2 : 0;
+        x1 = (c > 0 ? fl[m1][c > 0 ? c - 1 : 0] : fo[m][0]) ? pc : x1;
+        x2 = (c < COLS - 1 ? fl[m1][c < COLS - 1 ? c + 1 : c] : fo[m][1]) ? pc : x2;
+        y1 = fl[m][c] ? pc : y1;
+        y2 = fl[m2][c] ? pc : y2;
+      } else if (SP == 1) {
         auto side = [&](int bit) -> uint32_t {
           return (uint32_t)__builtin_amdgcn_sbfe((int)outer[SP == 1 ? (2 * r + bit) / 32 : 0],
                                                  (2 * r + bit) % 32, 1);
@@ -385,7 +413,6 @@ __device__ __forceinline__ void jacobi_tb_tile(
     // registers, and two sweeps bring every row back to where it was.  A strip
     // lives in ROWS + 1 rows of registers, without copies and without a second
     // strip of neighbour sums.
-    constexpr bool SMALL = ROWS * COLS <= 8;
     auto sweep = [&](auto upc, const float(&in)[ROWS][COLS], float(&out)[ROWS][COLS]) {
       constexpr bool UP = decltype(upc)::value;
       float prev[COLS], above[COLS];
