@@ -67,6 +67,7 @@ __device__ __forceinline__ int find_scene(const int* __restrict__ prefix, int S,
     if (x >= d.W || y >= d.H) continue;                                      \
     const long long pos = d.off + (long long)y * d.W + x;
 
+template <bool SKIP>
 __global__ void __launch_bounds__(256)
     kb_splats(const SceneDev* __restrict__ sc, int S,
               const int* __restrict__ prefix, int total, float2* __restrict__ u,
@@ -77,7 +78,7 @@ __global__ void __launch_bounds__(256)
     float dq = q ? q[pos] : 0.0f;
     for (int i = d.splat_begin; i < d.splat_end; ++i) {
       const Splat s = sp[i];
-      const float w = gaussian_weight(s, x, y, d.W, d.H);
+      const float w = gaussian_weight<SKIP>(s, x, y, d.W, d.H);
       v.x = v.x + s.ax * w;
       v.y = v.y + s.ay * w;
       dq = dq + s.dye * w;
@@ -264,6 +265,7 @@ struct nx_batch {
   std::vector<Splat> splats;  // sorted by scene
   Splat* d_splats = nullptr;
   size_t splat_cap = 0;
+  bool splats_skip = false;  // gaussian_weight's form, by the pairs of all scenes
   // prefix tables by tile width and height and sweeps (get_prefix)
   std::map<long long, std::pair<int*, int>> prefix;
   nx_params prm;
@@ -424,9 +426,14 @@ static int batch_step(nx_batch* b, float dt) {
   const int a = b->vcur;
   const bool merged = batch_step_merged(b);
   float* dq = b->dye[0] ? b->dye[b->dcur] : nullptr;
-  if (!b->splats.empty())
-    NXB_KERNEL(b, NX_TIME_SPLAT, kb_splats, tc, b->d_scenes, b->S, pc, tc,
-               b->vel[a], dq, b->d_splats);
+  if (!b->splats.empty()) {
+    if (b->splats_skip)
+      NXB_KERNEL(b, NX_TIME_SPLAT, kb_splats<true>, tc, b->d_scenes, b->S, pc, tc,
+                 b->vel[a], dq, b->d_splats);
+    else
+      NXB_KERNEL(b, NX_TIME_SPLAT, kb_splats<false>, tc, b->d_scenes, b->S, pc, tc,
+                 b->vel[a], dq, b->d_splats);
+  }
   if (merged) {
     NXB_KERNEL(b, NX_TIME_VORT_DIV, kb_fused<true>, tf, b->d_scenes, b->S, pf, tf,
                b->vel[a], b->mask[b->mcur], b->vel[1 - a], b->div, b->p[0], dt);
@@ -611,12 +618,17 @@ int nx_batch_set_step_splats(nx_batch* b, const float* rec, int n) {
                    });
   b->splats.clear();
   for (auto& d : b->scenes) d.splat_begin = d.splat_end = 0;
+  double pairs = 0.0, near = 0.0;
   for (size_t i = 0; i < v.size(); ++i) {
     SceneDev& d = b->scenes[v[i].first];
+    const double cells = (double)d.W * d.H;
+    pairs += cells;
+    near += cells * splat_share(v[i].second, d.W, d.H);
     if (d.splat_begin == d.splat_end) d.splat_begin = (int)i;
     d.splat_end = (int)i + 1;
     b->splats.push_back(v[i].second);
   }
+  b->splats_skip = near < SPLAT_SKIP_SHARE * pairs;
   NXB_HIP(hipStreamSynchronize(b->stream));
   if (b->splats.size() > b->splat_cap) {
     (void)hipFree(b->d_splats);

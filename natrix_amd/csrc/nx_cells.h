@@ -72,16 +72,33 @@ __device__ __forceinline__ float advect_dye_cell(
 
 // e2: w = float(exp(double(-(dx*dx + dy*dy) / (r*r)))).  Below -104 the
 // exponent's weight rounds to zero (exp(-104) < 2^-150), and beyond 105 r*r the
-// quotient is below that whatever its rounding: waves with no cell within 10.25
-// radii of the splat leave out the division and the float64 exponential, which
-// were the kernel's time (4096^2 bf16, 8 splats: 167 to 96 us).
+// quotient is below that whatever its rounding.  SKIP: waves with no cell within
+// 10.25 radii of the splat leave out the division and the float64 exponential,
+// which were the kernel's time (4096^2 bf16, 8 splats: 167 to 96 us).
+template <bool SKIP>
 __device__ __forceinline__ float gaussian_weight(const Splat& s, int x, int y,
                                                  int W, int H) {
   const float sx = s.px * (float)W, sy = s.py * (float)H;
   const float dx = sx - (float)x, dy = sy - (float)y;
   const float d2 = dx * dx + dy * dy, r2 = s.radius * s.radius;
-  if (d2 > 105.0f * r2) return 0.0f;
+  if (SKIP && d2 > 105.0f * r2) return 0.0f;
   return (float)exp((double)(-d2 / r2));
 }
+
+// Share of a W x H grid in the box of a splat's reach, 10.25 radii; a centre or
+// radius that is no number counts as all of it.
+inline float splat_share(const Splat& s, int W, int H) {
+  const float w = (float)W, h = (float)H, x = s.px * w, y = s.py * h;
+  const float reach = 10.25f * fabsf(s.radius);
+  const float bw = fminf(x + reach, w) - fmaxf(x - reach, 0.0f);
+  const float bh = fminf(y + reach, h) - fmaxf(y - reach, 0.0f);
+  return fmaxf(bw, 0.0f) / w * (fmaxf(bh, 0.0f) / h);
+}
+
+// SKIP pays while less than this share of the (cell, splat) pairs is within reach:
+// its branch makes a near pair cost 1.2 of what it costs without.  2048^2, 8
+// splats, us without / with at shares of 0.04, 0.36, 0.57, 0.76 and 1: 39.8 / 21.1,
+// 39.7 / 33.4, 39.9 / 38.7, 40.2 / 42.7, 40.4 / 47.8.
+constexpr float SPLAT_SKIP_SHARE = 0.55f;
 
 }  // namespace nx

@@ -92,7 +92,7 @@ struct SplatBatchM {
   Splat s[16];
 };
 
-template <class S>
+template <class S, bool SKIP>
 __global__ void __launch_bounds__(256)
     km_splats(typename S::s2* __restrict__ u, typename S::s1* __restrict__ q,
               int W, int H, SplatBatchM sb) {
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(256)
   float2 v = S::ld2(u, pos);
   float d = q ? S::ld(q, pos) : 0.0f;
   for (int i = 0; i < sb.n; ++i) {
-    const float w = gaussian_weight(sb.s[i], x, y, W, H);
+    const float w = gaussian_weight<SKIP>(sb.s[i], x, y, W, H);
     v.x = v.x + sb.s[i].ax * w;
     v.y = v.y + sb.s[i].ay * w;
     d = d + sb.s[i].dye * w;
@@ -288,9 +288,17 @@ static hipError_t splats_m(void* u, void* q, int W, int H, const Splat* sp, int 
   for (int i0 = 0; i0 < n; i0 += 16) {
     SplatBatchM sb;
     sb.n = n - i0 < 16 ? n - i0 : 16;
-    for (int i = 0; i < sb.n; ++i) sb.s[i] = sp[i0 + i];
-    km_splats<S><<<grid2d(W, H), dim3(BX, BY), 0, s>>>(
-        (typename S::s2*)u, (typename S::s1*)q, W, H, sb);
+    float share = 0.0f;
+    for (int i = 0; i < sb.n; ++i) {
+      sb.s[i] = sp[i0 + i];
+      share += splat_share(sb.s[i], W, H);
+    }
+    auto* us = (typename S::s2*)u;
+    auto* qs = (typename S::s1*)q;
+    if (share < SPLAT_SKIP_SHARE * sb.n)
+      km_splats<S, true><<<grid2d(W, H), dim3(BX, BY), 0, s>>>(us, qs, W, H, sb);
+    else
+      km_splats<S, false><<<grid2d(W, H), dim3(BX, BY), 0, s>>>(us, qs, W, H, sb);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

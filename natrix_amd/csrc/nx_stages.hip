@@ -260,6 +260,7 @@ struct SplatBatch {
   Splat s[16];
 };
 
+template <bool SKIP>
 __global__ void __launch_bounds__(256)
     k_gaussian(float2* __restrict__ u, float* __restrict__ q, int W, int H,
                SplatBatch sb) {
@@ -270,7 +271,7 @@ __global__ void __launch_bounds__(256)
   float d = q ? q[pos] : 0.0f;
   for (int i = 0; i < sb.n; ++i) {
     const Splat s = sb.s[i];
-    const float w = gaussian_weight(s, x, y, W, H);
+    const float w = gaussian_weight<SKIP>(s, x, y, W, H);
     v.x = v.x + s.ax * w;
     v.y = v.y + s.ay * w;
     d = d + s.dye * w;
@@ -379,8 +380,15 @@ hipError_t launch_gaussian_splats(float2* u, float* q, int W, int H,
   for (int i0 = 0; i0 < n; i0 += 16) {
     SplatBatch sb;
     sb.n = n - i0 < 16 ? n - i0 : 16;
-    for (int i = 0; i < sb.n; ++i) sb.s[i] = splats[i0 + i];
-    k_gaussian<<<grid2d(W, H), dim3(BX, BY), 0, s>>>(u, q, W, H, sb);
+    float share = 0.0f;
+    for (int i = 0; i < sb.n; ++i) {
+      sb.s[i] = splats[i0 + i];
+      share += splat_share(sb.s[i], W, H);
+    }
+    if (share < SPLAT_SKIP_SHARE * sb.n)
+      k_gaussian<true><<<grid2d(W, H), dim3(BX, BY), 0, s>>>(u, q, W, H, sb);
+    else
+      k_gaussian<false><<<grid2d(W, H), dim3(BX, BY), 0, s>>>(u, q, W, H, sb);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

@@ -121,3 +121,38 @@ def test_merged_reduced_storage_is_the_replay(gpu, storage, iters, corr):
         assert np.array_equal(sim.download("pressure32"), p32)
         assert np.array_equal(sim.download("divergence"), b)
         sim.destroy()
+
+
+@pytest.mark.parametrize("radius", [3.0, 6.0, 9.0, 40.0])
+def test_splats_whose_reach_covers_little_or_all(gpu, radius):
+    """Both forms of the weight, in a grid and in a batch: a reach of 10.25 radii is
+    a fifth of 160 x 120 cells, about half, most, and all of them."""
+    from natrix_amd.batch import BatchedScenes
+    w, h = 160, 120
+    rng = np.random.default_rng(6)
+    u = rng.standard_normal((h, w, 2)).astype(np.float32)
+    splats = [(0.3, 0.4, 0.5, -0.25, radius, 1.0), (0.6, 0.7, -1.5, 2.0, 1.3 * radius, 0.5)]
+    s32 = [tuple(np.float32(v) for v in s) for s in splats]
+    ref, q = F.gaussian_splat(u, np.zeros((h, w), np.float32), s32)
+    sim = FluidSimulator(w, h, dye=True)
+    sim.upload("velocity", u)
+    sim.add_splats(splats)
+    assert np.array_equal(sim.download("velocity").view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(sim.download("dye").view(np.uint32), q.view(np.uint32))
+    sim.destroy()
+    half = M.rounder("bf16")
+    sim = FluidSimulator(w, h, storage="bf16")
+    sim.upload("velocity", half(u))
+    sim.add_splats(splats)
+    assert np.array_equal(sim.download("velocity"), half(F.gaussian_splat(half(u), None, s32)[0]))
+    sim.destroy()
+    b, one = BatchedScenes([w, 50], [h, 40]), FluidSimulator(w, h)
+    b.upload(0, "velocity", u)
+    one.upload("velocity", u)
+    b.set_step_splats([(0,) + s for s in splats])
+    one.add_splats(splats)
+    b.update(1 / 60)
+    one.update(1 / 60)
+    assert np.array_equal(b.download(0, "velocity"), one.download("velocity"))
+    b.destroy()
+    one.destroy()
