@@ -190,7 +190,7 @@ int nx_prolong_line_search(nx_sim* sim, int factor, const float* coarse,
                            const uint8_t* coarse_mask, double* out);
 /* smoothing of the coarse correction problem L e = rc on a Wc x Hc grid
  * (at most 128 x 128; device buffers as written by nx_restrict_residual),
- * e[Hc*Wc] updated in place, one launch on the simulator's stream:
+ * e[Hc*Wc] updated in place, enqueued on the simulator's stream:
  * lambda_min <= 0: `iterations` Jacobi sweeps (the fine sweep's operator);
  * 0 < lambda_min < 8: `iterations` Chebyshev iterations of the same
  * operator on [lambda_min, 8] (-L has its spectrum in [0, 8]) */

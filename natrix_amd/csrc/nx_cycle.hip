@@ -450,13 +450,19 @@ __global__ void __launch_bounds__(256)
 constexpr int CT_ROWS = 3, CT_WAVES = 16, CT_COLS = 1;
 // iterations a launch: the halos of 20 leave 6 rows of a tile's 48, which pays
 // while all tiles run at once (two workgroups a CU), else 12
-constexpr int CT_T = 20, CT_T_MANY = 12, CT_TILES = 512;
+constexpr int CT_T = 20, CT_T_MANY = 12, CT_TILES = 512, CT_ASIDE = 256;
 constexpr int CB_T = 12;  // plain operator: up to here one resident workgroup does it
 
 template <bool FACES>
 __global__ void __launch_bounds__(64 * CT_WAVES)
     k_coarse_cheb_tile(nx::jt::ChebArgs a, ChebCoef cf) {
   nx::jt::cheb_tile<CT_ROWS, CT_WAVES, CT_COLS, FACES, false>(a, cf, (int)blockIdx.x);
+}
+
+static __global__ void __launch_bounds__(256)
+    k_copy(const float* __restrict__ in, float* __restrict__ out, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = in[i];
 }
 
 namespace nx {
@@ -477,9 +483,14 @@ int launch_coarse_smooth(hipStream_t st, int Wc, int Hc, float* e, const float* 
     const int most = nx::jt::cheb_tiles(Wc, Hc, EX, EY, CT_T + 1) <= CT_TILES ? CT_T : CT_T_MANY;
     ChebRecurrence rec(lambda_min);
     int launches = (iterations + most - 1) / most;
-    // e is the first launch's input and the last one's output: one launch does
-    // only where one tile holds the grid
-    if (launches == 1 && nx::jt::cheb_tiles(Wc, Hc, EX, EY, 1) > 1) launches = 2;
+    // e is the first launch's input and the last one's output.  A single launch of
+    // several tiles, which read their neighbours' cells, therefore writes to ws and
+    // is copied; on a grid of more than a tile a CU two launches of half the
+    // iterations and halo cost no more (128 x 128, 5 and 12 iterations: 9.9 and 11.8
+    // us against 13.3 and 15.4; 512 x 512, 12: equal)
+    const int tiles = nx::jt::cheb_tiles(Wc, Hc, EX, EY, iterations + 1);
+    const bool aside = launches == 1 && tiles > 1 && tiles <= CT_ASIDE;
+    if (launches == 1 && tiles > CT_ASIDE) launches = 2;
     int done = 0, cur = 0;
     for (int l = 0; l < launches; ++l) {
       const int T = (iterations - done + launches - l - 1) / (launches - l);
@@ -488,7 +499,7 @@ int launch_coarse_smooth(hipStream_t st, int Wc, int Hc, float* e, const float* 
       ChebCoef cf{};
       rec.next(first, T + first, cf);
       const nx::jt::ChebArgs a{first ? e : set[cur][0], set[cur][1], set[cur][2], rc, mc, faces,
-                               last ? e : out[0], last ? nullptr : out[1], out[2], Wc, Hc, T,
+                               last && !aside ? e : out[0], last ? nullptr : out[1], out[2], Wc, Hc, T,
                                first ? 1 : 0, T + (first ? 1 : 0), rec.theta, nullptr, nullptr,
                                nullptr};
       const int grid = nx::jt::cheb_tiles(Wc, Hc, EX, EY, a.halo);
@@ -500,6 +511,11 @@ int launch_coarse_smooth(hipStream_t st, int Wc, int Hc, float* e, const float* 
         return set_error(NX_ERR_HIP, "coarse smoother launch failed");
       cur = first ? 0 : 1 - cur;
       done += T;
+    }
+    if (aside) {
+      k_copy<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(ws, e, (int)n);
+      if (hipGetLastError() != hipSuccess)
+        return set_error(NX_ERR_HIP, "coarse smoother launch failed");
     }
   } else if (lambda_min > 0.0f) {
     k_coarse_smooth<true><<<1, 1024, 0, st>>>(e, rc, mc, Wc, Hc, iterations, lambda_min);

@@ -194,10 +194,9 @@ int conv3x3_fwd_tiled(const void* x, const void* wt, const float* bias, void* y,
 
 // Coarse smoothing of L e = rc on a Wc x Hc (<= 128 x 128) grid: Jacobi
 // sweeps (lambda_min <= 0) or Chebyshev on [lambda_min, 8]; more than 12
-// Chebyshev iterations run on 2D tiles over many workgroups (at least two
-// launches where there is more than one tile: e is read by the first and written
-// by the last) and need ws = 6 Wc Hc floats.  faces (2 Wc Hc floats, east then south weights):
-// the face-weighted operator, always tiled, Chebyshev only.
+// Chebyshev iterations run on 2D tiles over many workgroups and need ws = 6 Wc Hc
+// floats.  faces (2 Wc Hc floats, east then south weights): the face-weighted
+// operator, always tiled, Chebyshev only.
 int launch_coarse_smooth(hipStream_t st, int Wc, int Hc, float* e, const float* rc,
                          const uint8_t* mc, int iterations, float lambda_min, float* ws,
                          const float* faces = nullptr);
