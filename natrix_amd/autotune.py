@@ -16,6 +16,15 @@ and is cached under ``batch_key(sizes)`` for ``BatchedScenes``.
 The fine Chebyshev smoother of the learned cycle is tuned per grid as well
 (``tune_smoother``: tile and streaming launch shapes, timed on the
 smoothing call the cycle makes) and cached under "cheb".
+
+The entries in the repository were chosen by whole steps of three simulators
+taking turns, where the last blocks of one launch run beside the next
+simulator's first; the tuner times the sweeps of one simulator alone and may
+pick another tile (2048 x 2048: 12 sweeps a launch, 2.12 us each, over the
+table's 13, 2.26).  ``us_per_sweep`` and ``us_per_iteration`` (72 a call) are its
+figures for the tiles in the table; storing a new choice overwrites them.
+Reduced storage is not tuned by the command line: its sweeps per launch are
+fixed (``lookup``) and its shapes were chosen by whole steps.
 """
 from __future__ import annotations
 
@@ -31,7 +40,7 @@ ARCH = "gfx950"
 SHAPES = [(4, 8, 1), (4, 16, 1), (8, 8, 1), (8, 16, 1), (16, 8, 1), (2, 8, 2), (2, 16, 2),
           (4, 4, 2), (4, 8, 2), (4, 16, 2), (8, 4, 2), (8, 8, 2), (8, 16, 2), (16, 4, 1),
           (16, 4, 2), (16, 8, 2)]
-KS = (2, 4, 6, 8, 10, 12, 14, 16, 20, 24, 28)
+KS = (2, 4, 6, 8, 10, 12, 13, 14, 16, 20, 24, 28)
 DEFAULT = (6, 4, 8, 2)
 
 
@@ -233,7 +242,7 @@ def store_step_timed(W, H, tile, ms_per_step, dtype):
 # NX_CHEB_SHAPES in csrc/nx_cheb.hip) and streaming kernels (seg > 0;
 # NX_STREAM_SHAPES in csrc/nx_stream.hip)
 CHEB_SHAPES = [(2, 16, 2), (4, 8, 2), (4, 16, 2), (4, 16, 1), (8, 8, 1), (8, 16, 1), (8, 8, 2)]
-CHEB_KS = (4, 6, 8, 10, 12, 16, 20, 25)
+CHEB_KS = (4, 6, 8, 10, 12, 13, 15, 16, 20, 25)
 STREAM_SHAPES = [(4, 8, 2), (2, 16, 2), (4, 16, 2), (8, 8, 2), (8, 4, 2)]
 STREAM_KS = (8, 12, 16)
 STREAM_SEGS = (48, 80, 112, 144, 208)
