@@ -250,6 +250,7 @@ static int bfail(int code, const std::string& m) { return nx::set_error(code, m)
 struct nx_batch {
   int S = 0;
   std::vector<int> W, H;
+  long long stage_tiles = 0;  // tiles of the stages' kernel, all scenes
   std::vector<long long> off;
   long long cells = 0;
   hipStream_t stream = nullptr;
@@ -365,20 +366,20 @@ struct BTime {
     t_.end();                                                         \
   } while (0)
 
-// project: the last launch also projects vel[1 - vcur] and writes the next masks
-static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c, bool project = false) {
+// u != nullptr: the last launch also projects u in place and writes the next masks
+static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c, float2* u = nullptr) {
   c.k = jacobi_even_k(sweeps, c.k);
   while (sweeps > 0) {
     JacobiCfg cc = c;
     if (sweeps < cc.k) cc.k = sweeps;
-    const bool last = project && sweeps == cc.k;
+    const bool last = u && sweeps == cc.k;
     int* pre;
     int total;
     NXB_TRY(get_prefix(b, 64 * cc.cols, cc.rows * cc.waves, cc.k + (last ? 1 : 0), &pre, &total));
     NXB_TIMED(b, NX_TIME_JACOBI,
               launch_batch_jacobi(b->d_scenes, b->S, pre, total, b->p[b->pcur],
                                   b->div, b->mask[b->mcur], b->p[1 - b->pcur], cc,
-                                  last ? b->vel[1 - b->vcur] : nullptr, b->mask[1 - b->mcur],
+                                  last ? u : nullptr, b->mask[1 - b->mcur],
                                   b->stream));
     b->pcur ^= 1;
     sweeps -= cc.k;
@@ -386,16 +387,28 @@ static int batch_jacobi(nx_batch* b, int sweeps, JacobiCfg c, bool project = fal
   return NX_OK;
 }
 
-// one launch for the advection and the stages up to the first sweep, and the
-// projection in the last Jacobi launch, unless the kernels are timed one by one
-// or there is no further sweep
+// the projection in the last Jacobi launch, and in small batches one launch for
+// the advection and the stages up to the first sweep (batch_step_advects), unless
+// the kernels are timed one by one or there is no further sweep
 static bool batch_step_merged(const nx_batch* b) { return !b->timing && b->prm.iterations > 1; }
+
+// The advection joins the stages' kernel up to three of its tiles a CU, where a
+// launch less counts: us a step of 20 sweeps merged / apart with 256 tiles (16
+// scenes of 128^2) 38.1 / 38.9, 824 (20 uneven scenes) 59.1 / 57.6, 1024 (one of
+// 1024^2) 55.1 / 52.5, 8192 298 / 275, 24 000 (the 64 benchmark scenes) 1272 / 1177.
+// Beyond, its gathers take longer than the pass they save: 571 us in the last,
+// where the two kernels take 267 + 230.
+constexpr int BATCH_ADVECT_TILES = 768;
+
+static bool batch_step_advects(const nx_batch* b) {
+  return batch_step_merged(b) && b->stage_tiles <= BATCH_ADVECT_TILES;
+}
 
 static int batch_step_launches(const nx_batch* b) {
   const int sweeps = b->prm.iterations - 1;
   const int jacobi = sweeps > 0 ? (sweeps + b->prm.jacobi_k - 1) / b->prm.jacobi_k : 0;
-  return (batch_step_merged(b) ? 1 : 3) + jacobi + (b->splats.empty() ? 0 : 1) +
-         (b->dye[0] ? 1 : 0);
+  return (!batch_step_merged(b) ? 3 : batch_step_advects(b) ? 1 : 2) + jacobi +
+         (b->splats.empty() ? 0 : 1) + (b->dye[0] ? 1 : 0);
 }
 
 // every prefix table a step needs (no allocation inside a capture)
@@ -424,7 +437,7 @@ static int batch_step(nx_batch* b, float dt) {
   NXB_TRY(get_prefix(b, 64, 4, 0, &pc, &tc));
   NXB_TRY(get_prefix(b, fused::TX, fused::TY, 0, &pf, &tf));
   const int a = b->vcur;
-  const bool merged = batch_step_merged(b);
+  const bool merged = batch_step_merged(b), advects = batch_step_advects(b);
   float* dq = b->dye[0] ? b->dye[b->dcur] : nullptr;
   if (!b->splats.empty()) {
     if (b->splats_skip)
@@ -434,7 +447,7 @@ static int batch_step(nx_batch* b, float dt) {
       NXB_KERNEL(b, NX_TIME_SPLAT, kb_splats<false>, tc, b->d_scenes, b->S, pc, tc,
                  b->vel[a], dq, b->d_splats);
   }
-  if (merged) {
+  if (advects) {
     NXB_KERNEL(b, NX_TIME_VORT_DIV, kb_fused<true>, tf, b->d_scenes, b->S, pf, tf,
                b->vel[a], b->mask[b->mcur], b->vel[1 - a], b->div, b->p[0], dt);
   } else {
@@ -445,12 +458,14 @@ static int batch_step(nx_batch* b, float dt) {
   }
   b->pcur = 0;
   JacobiCfg c{P.jacobi_k, P.jacobi_rows, P.jacobi_waves, P.jacobi_cols};
-  NXB_TRY(batch_jacobi(b, P.iterations - 1, c, merged));
+  // where the stages left the velocity, and a merged step projects it in place
+  const int v = advects ? 1 - a : a;
+  NXB_TRY(batch_jacobi(b, P.iterations - 1, c, merged ? b->vel[v] : nullptr));
   if (!merged)
     NXB_KERNEL(b, NX_TIME_PROJECT, kb_subgrad, tc, b->d_scenes, b->S, pc, tc,
                b->vel[a], b->p[b->pcur], b->mask[b->mcur], b->vel[1 - a],
                b->mask[1 - b->mcur]);
-  b->vcur = 1 - a;
+  b->vcur = merged ? v : 1 - a;
   b->mcur ^= 1;
   if (b->dye[0]) {
     NXB_KERNEL(b, NX_TIME_DYE, kb_advect_dye, tc, b->d_scenes, b->S, pc, tc,
@@ -485,6 +500,8 @@ int nx_batch_create(int n, const int* widths, const int* heights, int with_dye,
     b->H.push_back(heights[s]);
     b->off.push_back(cells);
     cells += (long long)widths[s] * heights[s];
+    b->stage_tiles += (long long)((widths[s] + fused::TX - 1) / fused::TX) *
+                      ((heights[s] + fused::TY - 1) / fused::TY);
   }
   b->cells = cells;
   nx_default_params(&b->prm);
@@ -689,7 +706,7 @@ int nx_batch_update(nx_batch* b, float dt) {
     pcn ^= 1;
   }
   b->pcur = pcn;
-  b->vcur ^= 1;
+  if (!batch_step_merged(b) || batch_step_advects(b)) b->vcur ^= 1;
   b->mcur ^= 1;
   if (dye) b->dcur ^= 1;
   return NX_OK;

@@ -107,6 +107,36 @@ def test_batch(gpu, iters):
     g.destroy()
 
 
+@pytest.mark.parametrize("sides,tiles", [((512, 512, 512), 768), ((512, 512, 512, 40), 771)])
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_on_either_side_of_the_advecting_form(gpu, sides, tiles, graph):
+    """The last batch whose stages advect and the first whose do not, which leaves
+    the velocity in the other buffer: against the timed batch's separate launches."""
+    assert sum(-(-s // 64) * -(-s // 16) for s in sides) == tiles
+    rng = np.random.default_rng(5)
+    from natrix_amd.batch import BatchedScenes
+    bs = [BatchedScenes(sides, dye=True) for _ in range(2)]
+    for i, s in enumerate(sides):
+        u = rng.uniform(-0.5, 0.5, (s, s, 2)).astype(np.float32)
+        solid = rng.random((s, s)) < 0.03
+        for b in bs:
+            b.upload(i, "velocity", u)
+            b.set_obstacle_map(i, solid)
+    for b in bs:
+        b.set_params(iterations=40, vorticity=0.3, viscosity=0.0, jacobi_tile=(4, 8, 8, 1))
+    bs[0].use_graph = graph
+    bs[1].set_timing(True)
+    for step in range(5):
+        for b in bs:
+            b.update(1 / 60)
+        for i in range(len(sides)):
+            for f in ("velocity", "pressure", "dye"):
+                _same(*(b.download(i, f) for b in bs), step, i, f)
+    assert bs[0].graph_replays == (5 if graph else 0)
+    for b in bs:
+        b.destroy()
+
+
 def test_benchmark_batch(gpu):
     import bench
     got = []
