@@ -10,9 +10,10 @@
 // 12+20+(16)+13+4+13 bytes the separate passes move.  With the advection in
 // front (the merged step) the block makes the advected velocity itself, halo
 // included, instead of reading what a pass of its own wrote: 25 bytes a cell
-// instead of 42, for 1.5 times the gathers.  Bound by the gathers' latency:
-// 2048^2 50 us where the two passes took 51, 4096^2 bf16 137 us against 167,
-// 128^2 9 us against 12.5.
+// instead of 42, for 1.5 times the gathers.  Bound by the gathers' latency, so
+// that at 2048^2 the bytes saved buy little (48.0 us for 20.7 + 28.9) and the gain
+// is a launch less (128^2 9 us against 12.5) and, in bf16, the conversions of the
+// stored velocity (4096^2 137 us against 167).
 //
 // Each LDS slot holds its stage's value at the CLAMPED grid coordinate of the
 // slot, and neighbours are looked up at clamp(c +- 1) as common.sh:14-17 does,

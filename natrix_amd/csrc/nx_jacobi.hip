@@ -17,13 +17,15 @@
 // neighbours (Poisson.comp:32-35) are both "use the centre value".  A wave
 // takes the sweep's select-free form when its strip touches neither.
 //
-// Bound: with many tiles, VALU issue (a wave64 addition takes 2 cycles when
-// two waves or more share a SIMD, a DPP one 4: 12 cycles per pair of columns
-// and row) and, between blocks, the load of the next tile; with few, the
-// exchange's latency.  Per sweep, launch gaps included: 2048^2 (13, 8, 8, 2)
-// 1.97 us (2.99 before the in-grid tiles, masks on demand and the register
-// walk, with tile (10, 8, 8, 1)), 4096^2 (20, 16, 8, 2) 5.4 us (8.76), 1024^2
-// (20, 4, 16, 2) 1.07 us (1.48), 256^2 (24, 4, 16, 1) 0.48 us (0.69).
+// Bound: latency, of the load and then of one LDS exchange and barrier a sweep,
+// with the waves next to solids setting a round's pace.  2048^2 on (13, 8, 8, 2)
+// is one round of 361 blocks on 256 CUs: 0.33 of its time issues VALU (per row and
+// pair of columns ten instructions, two of them lane shifts at 4 cycles, the
+// others at 2: 24 cycles), 0.36 of the HBM peak moves its bytes, and 41 % of the
+// wave cycles wait.  us per sweep of one simulator, launches of k sweeps (the
+// tuner's figure; before the in-grid tiles and the register walk, on the tiles
+// chosen then): 2048^2 (13, 8, 8, 2) 2.26 (2.99), 4096^2 (20, 16, 8, 2) 5.66 (8.76),
+// 1024^2 (20, 4, 16, 2) 1.10 (1.48), 256^2 (24, 4, 16, 1) 0.56 (0.69).
 #include "nx_jacobi_tile.h"
 #include "nx_kernels.h"
 

@@ -9,7 +9,7 @@ namespace nx {
 namespace jt {
 
 // Waves per SIMD asked of the compiler for a tile kernel of CELLS cells
-// per lane (amdgpu_waves_per_eu; 1 leaves it free).  Jacobi: what the strip,
+// per lane (amdgpu_waves_per_eu).  Jacobi: what the strip,
 // its right-hand side and, next to solids, its masks fit in without spills in
 // the sweeps; asked for one step more (8 for 16 cells, 5 for 32) the spills
 // cost more than the waves give (2048^2, (12, 8, 8, 2): 1.96 to 2.27 us per

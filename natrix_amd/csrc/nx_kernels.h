@@ -56,13 +56,13 @@ hipError_t launch_gaussian_splats(float2* u, float* q, int W, int H,
                                   const Splat* splats, int n, hipStream_t s);
 
 // ---- fused fast path ---------------------------------------------------
-// curl + confinement (+ viscosity) + divergence + first Jacobi sweep from a
-// zero guess: writes the projected-step velocity input, b and p1.
 // advection (walls on its reads) and launch_fused_vort_div in one pass
 hipError_t launch_advect_vort_div(const float2* uin, const uint8_t* mask, float2* uout,
                                   float* div, float* p1, int W, int H, float dt, float speed,
                                   float diss, BcParams bc, float scale, int viscous, float alpha,
                                   float rbeta, hipStream_t s);
+// curl + confinement (+ viscosity) + divergence + first Jacobi sweep from a
+// zero guess: writes the projected-step velocity input, b and p1.
 hipError_t launch_fused_vort_div(const float2* uin, const uint8_t* mask,
                                  float2* uout, float* div, float* p1, int W,
                                  int H, float dt, float scale, int viscous,
@@ -237,13 +237,13 @@ hipError_t launch_m_advect_fused(int st, const void* uin, const uint8_t* mask, v
 hipError_t launch_m_fused(int st, const void* uin, const uint8_t* mask, void* uout,
                           void* div, void* p1, int W, int H, float dt, float scale,
                           int viscous, float alpha, float rbeta, hipStream_t s);
-// corr = false: k sweeps, p stored in `st`; corr = true: float32 residual
-// correction (1 residual pass + k-1 sweeps), float32 p + e to pout32
 // the correction launch (launch_m_jacobi with corr) and the projection of u with
 // its pressure in place, one launch
 hipError_t launch_m_correct_project(int st, const void* pin, const void* b, const uint8_t* mask,
                                     float* pout32, void* u, uint8_t* mask_next, int W, int H,
                                     JacobiCfg c, hipStream_t s);
+// corr = false: k sweeps, p stored in `st`; corr = true: float32 residual
+// correction (1 residual pass + k-1 sweeps), float32 p + e to pout32
 hipError_t launch_m_jacobi(int st, const void* pin, const void* b, const uint8_t* mask,
                            void* pout, float* pout32, int W, int H, JacobiCfg c,
                            bool corr, hipStream_t s);
