@@ -61,43 +61,54 @@ def _load():
         return {}
 
 
+def _nearest(table, W, H):
+    """Tile of the grid's own entry, else of the nearest cell count's, else None."""
+    if f"{W}x{H}" in table:
+        return tuple(table[f"{W}x{H}"]["tile"])
+    best, dist = None, None
+    for k, v in table.items():
+        if k.startswith("batch"):
+            continue
+        w, h = (int(t) for t in k.split("x"))
+        d = abs((w * h) - W * H)
+        if dist is None or d < dist:
+            best, dist = tuple(v["tile"]), d
+    return best
+
+
 def lookup(W, H, dtype="f32"):
     """Tuned tile for a W x H grid with `dtype` storage: the entry of that
     storage for the grid, else the one with the nearest cell count, else (a
     storage without entries) the float32 one, else the built-in default.
-    Reduced storage has its own entries because its sweeps per launch are part
-    of its result: the pressure is rounded to storage after every launch, so
-    they stay what they were (12 to 256^2, 16 at 512^2, 10 beyond) and only the
-    tile's shape is tuned."""
+    Reduced storage has its own entries, of which only the shape counts: its
+    sweeps per launch are part of its result, since the pressure is rounded to
+    storage after every launch, and so the grid's (grid_sweeps)."""
     data = _load().get(ARCH, {})
-    for table in (data.get(dtype, {}), data.get("f32", {})):
-        key = f"{W}x{H}"
-        if key in table:
-            return tuple(table[key]["tile"])
-        best, dist = None, None
-        for k, v in table.items():
-            if k.startswith("batch"):
-                continue
-            w, h = (int(t) for t in k.split("x"))
-            d = abs((w * h) - W * H)
-            if dist is None or d < dist:
-                best, dist = tuple(v["tile"]), d
-        if best is not None:
-            return best
-    return DEFAULT
+    tile = (_nearest(data.get(dtype, {}), W, H) or _nearest(data.get("f32", {}), W, H) or
+            DEFAULT)
+    if dtype == "f32":
+        return tile
+    fixed = (grid_sweeps(W, H),) + tile[1:]
+    return fixed if supported(*fixed) else tile
 
 
-# sides of the grids whose check interval is known, and the sweeps it is made
-# of (nearest cell count; the first of two equally near)
-CHECK_UNITS = ((1024, 10), (256, 12), (512, 16))
+# sweeps that belong to a grid and not to a tile, by the side of the square with
+# the nearest cell count (the first of two equally near)
+GRID_SWEEPS = ((1024, 10), (256, 12), (512, 16))
+
+
+def grid_sweeps(W, H):
+    """Sweeps per launch of reduced storage on a W x H grid, and the unit of a
+    tolerance solve's check interval: both decide results, so a retune of the
+    tiles may not move them."""
+    return min(GRID_SWEEPS, key=lambda t: abs(t[0] * t[0] - W * H))[1]
 
 
 def check_interval(W, H, check_every):
     """Sweeps between two residual checks of a tolerance solve on a tuned
     tile: `check_every`, rounded up to whole units of the grid.  Where a solve
-    stops is part of its result, so the unit belongs to the grid and not to
-    the table's tile, whose sweeps per launch a retune may change."""
-    _, unit = min(CHECK_UNITS, key=lambda t: abs(t[0] * t[0] - W * H))
+    stops is part of its result."""
+    unit = grid_sweeps(W, H)
     return -(-check_every // unit) * unit
 
 

@@ -23,6 +23,13 @@ def test_interval_whatever_the_tile(size, unit):
                 assert -(-every // d) * d == want, (every, k, d)
 
 
+@pytest.mark.parametrize("size,unit", sorted(UNIT.items()))
+def test_reduced_storage_keeps_its_sweeps(size, unit):
+    for dtype in ("bf16", "f16"):
+        tile = autotune.lookup(*size, dtype)
+        assert tile[0] == unit and autotune.supported(*tile)
+
+
 def test_default_interval_keeps_the_tuned_launches():
     for side in (96, 128, 256, 512, 1024, 2048, 4096):
         k = autotune.lookup(side, side)[0]
