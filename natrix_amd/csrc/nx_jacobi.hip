@@ -19,9 +19,9 @@
 //
 // Bound: latency, of the load and then of one LDS exchange and barrier a sweep,
 // with the waves next to solids setting a round's pace.  2048^2 on (13, 8, 8, 2)
-// is one round of 361 blocks on 256 CUs: 0.33 of its time issues VALU (per row and
+// is one round of 361 blocks on 256 CUs: 0.34 of its time issues VALU (per row and
 // pair of columns ten instructions, two of them lane shifts at 4 cycles, the
-// others at 2: 24 cycles), 0.36 of the HBM peak moves its bytes, and 41 % of the
+// others at 2: 24 cycles), 0.37 of the HBM peak moves its bytes, and 40 % of the
 // wave cycles wait.  us per sweep of one simulator, launches of k sweeps (the
 // tuner's figure; before the in-grid tiles and the register walk, on the tiles
 // chosen then): 2048^2 (13, 8, 8, 2) 2.26 (2.99), 4096^2 (20, 16, 8, 2) 5.66 (8.76),

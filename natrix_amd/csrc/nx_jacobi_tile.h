@@ -12,8 +12,8 @@ namespace jt {
 // per lane (amdgpu_waves_per_eu).  Jacobi: what the strip,
 // its right-hand side and, next to solids, its masks fit in without spills in
 // the sweeps; asked for one step more (8 for 16 cells, 5 for 32) the spills
-// cost more than the waves give (2048^2, (12, 8, 8, 2): 1.96 to 2.27 us per
-// sweep).
+// cost more than the waves give (2048^2, three simulators in turn: (12, 8, 8, 2)
+// 1.51 to 1.58 us per sweep, (13, 8, 8, 2) 1.42 to 1.47).
 template <int CELLS>
 constexpr int jacobi_waves_per_eu() {
   return CELLS <= 8 ? 8 : CELLS <= 16 ? 6 : CELLS <= 32 ? 4 : 2;
